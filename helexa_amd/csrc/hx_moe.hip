@@ -764,6 +764,14 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
         join.armed = false;
         HX_HIP(hipStreamWaitEvent(s, m->ev_join, 0));
       }
+    } else if (prefill_bf16_ok(p.ea)) {
+      // bf16 weights on MFMA, f32 h as three bf16 planes
+      tm_ext(m, SLOT_GATE_UP, s);
+      HX_HIP(launch_gate_up_bf16(p.ea, s));
+      tm_ext_done(m, SLOT_GATE_UP);
+      tm_ext(m, SLOT_DOWN, s);
+      HX_HIP(launch_down_bf16(p.ea, s));
+      tm_ext_done(m, SLOT_DOWN);
     } else {
       // generic GEMVs: the m <= 64 slots read the f32 d q of the tokens' and
       // then of their rows of h's Q8 codes (GGUF weights)

@@ -35,16 +35,11 @@
 // B[8(l/16)+i][l%16] and D rows 4(l/16)+i of column l%16). The next chunk's
 // global loads are issued before the current chunk's MFMAs. 52 KB of LDS per
 // workgroup: three workgroups per CU.
-#include "hx_internal.h"
+#include "hx_prefill_dev.h"
 #include <type_traits>
 
 namespace hx {
 
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-constexpr int PM = 64;            // rows of an M tile
 constexpr int PKC = 128;          // K chunk (f16 elements)
 constexpr int PLD = PKC + 8;      // LDS row pitch (f16 elements)
 
@@ -216,32 +211,6 @@ struct ARaw {
 
 
 HX_DEV f16x8_t frag(const uint16_t* base) { return __builtin_bit_cast(f16x8_t, *(const uint4*)base); }
-
-// the M tile of a workgroup (expert, first permuted row, rows): from the
-// dispatch list, or for a shared-expert-only launch computed from T; false if
-// the workgroup has no tile (past the end, or a tile the launch skips). TS is
-// the launch's tile selection (HX_TILES_*), a template parameter so that each
-// selection is a kernel of its own name in traces and counter runs.
-// m: the rows of the expert's call (the reference's arm: m <= HX_QUANT_M
-// quantised activations, else f16)
-template <int TS>
-HX_DEV bool get_tile(const ExpertArgs& a, int tile, int& e, int& p0, int& rows, int& m) {
-  if (TS == HX_TILES_SHARED) {
-    const int m0 = tile * PM;
-    if (m0 >= a.T) return false;
-    e = a.E;
-    p0 = a.F + m0;
-    rows = min(PM, a.T - m0);
-    m = a.T;
-    return true;
-  }
-  if (tile >= a.counts[1]) return false;
-  m = a.tiles[4 * tile + 0];
-  e = a.tiles[4 * tile + 1];
-  p0 = a.tiles[4 * tile + 2];
-  rows = a.tiles[4 * tile + 3];
-  return !(TS == HX_TILES_ROUTED && e == a.E);
-}
 
 // ---------------------------------------------------------------- Q4_K gate/up, streamed
 // k_gate_up_q4k<FPW, NW>: the gate/up GEMM for Q4_K weights, operands

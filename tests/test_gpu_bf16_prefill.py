@@ -1,0 +1,26 @@
+"""bf16 experts in prefill (the MFMA grouped GEMMs): tiles of 1 to 64 rows and
+their remainders, every width the kernels' chunks allow from the smallest, with
+and without a shared expert, both routings, against the oracle's exact block.
+
+Tolerance: products are exact and summed in f32 (terms of order 2^-24), so the
+distance is the bf16 rounding of the weighted expert rows and of the output,
+each at most 2^-9 of the value: max-normwise |y - ref| <= 2^-9 (sum over the
+rows of a token of |row| + |y|). The rows of a token partly cancel in y; the sum
+of their magnitudes is below 4 max|y| over these inputs, so 5 * 2^-9 < 1e-2
+(TOL_BF16)."""
+import pytest
+
+from oracle import oracle as O
+from tests.test_gpu_branches import TOL_BF16, Blk
+
+pytestmark = pytest.mark.gpu
+
+
+# (H, E, k, I, shared, renormalised): rows of an expert's call follow from T k / E
+@pytest.mark.parametrize("H,E,k,I,shared,norm", [(256, 4, 2, 256, 256, True), (2048, 64, 8, 512, 512, True),
+                                                 (1536, 8, 4, 768, 0, True), (768, 16, 4, 1024, 1024, False)])
+@pytest.mark.parametrize("T", [9, 31, 33, 130])
+def test_bf16_prefill_tiles(H, E, k, I, shared, norm, T):
+    from helexa_amd import synth
+    b = Blk(H, E, k, I, shared, norm, synth.FMT_BF16, O.BF16, 500 + H + E)
+    b.check(b.x(T, seed=T), TOL_BF16, tag=f"bf16 prefill H{H} I{I} T={T}")
