@@ -231,6 +231,9 @@ bool prefill_mfma_ok(const ExpertArgs& a);   // bf16 activations, GGUF experts: 
 hipError_t launch_x_to_f16(const ExpertArgs& a, hipStream_t s);       // tokens -> f16 for the MFMA kernels
 hipError_t launch_gate_up_mfma(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_down_mfma(const ExpertArgs& a, hipStream_t s);
+// Q8_0 weights; grid as the launches above
+hipError_t launch_gate_up_q8(const ExpertArgs& a, dim3 grid, hipStream_t s);
+hipError_t launch_down_q8(const ExpertArgs& a, dim3 grid, hipStream_t s);
 bool prefill_bf16_ok(const ExpertArgs& a);   // bf16 activations, bf16 experts: MFMA grouped GEMMs
 hipError_t launch_gate_up_bf16(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_down_bf16(const ExpertArgs& a, hipStream_t s);

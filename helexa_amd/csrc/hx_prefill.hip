@@ -104,39 +104,6 @@ struct PRaw<HX_Q4_K> {
   }
 };
 
-// Q8_0 planar: part pt holds blocks 4 kc + 2 pt and + 1 (64 int8 + 2 scales)
-template <>
-struct PRaw<HX_Q8_0> {
-  uint4 q[4];
-  uint32_t d;
-  HX_DEV void load(const uint8_t* mat, int R, int K, int row, int kc, int pt) {
-    const int b0 = 4 * kc + 2 * pt;
-    const uint4* p = (const uint4*)(mat + (int64_t)row * K + 32 * b0);
-#pragma unroll
-    for (int v = 0; v < 4; v++) q[v] = p[v];
-    d = *(const uint32_t*)((const uint16_t*)(mat + (int64_t)R * K) + (int64_t)row * (K / 32) + b0);
-  }
-  HX_DEV void to_lds(uint16_t* dst) const {
-    const h2_t off = h2s(-1152.0f);
-    uint4* o = (uint4*)dst;
-#pragma unroll
-    for (int b = 0; b < 2; b++) {
-      const h2_t s = h2s(f16_to_f32((uint16_t)(d >> (16 * b))));
-      const uint32_t w[8] = {q[2 * b].x, q[2 * b].y, q[2 * b].z, q[2 * b].w,
-                             q[2 * b + 1].x, q[2 * b + 1].y, q[2 * b + 1].z, q[2 * b + 1].w};
-      uint32_t r[16];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const uint32_t u = w[j] ^ 0x80808080u;                     // int8 -> q + 128
-        r[2 * j] = mul_pair(__builtin_amdgcn_perm(u, 0x64646464u, 0x00060004u), s, off);
-        r[2 * j + 1] = mul_pair(__builtin_amdgcn_perm(u, 0x64646464u, 0x00070005u), s, off);
-      }
-#pragma unroll
-      for (int v = 0; v < 4; v++) o[4 * b + v] = make_uint4(r[4 * v], r[4 * v + 1], r[4 * v + 2], r[4 * v + 3]);
-    }
-  }
-};
-
 // Q6_K planar: chunk kc = half n = kc & 1 of superblock kc >> 1 (quarters
 // s = 0..3 of 32 elements each); part pt holds quarters pt and pt + 2: ql bytes
 // 32 pt .. +31 of the half (low / high nibble) and the half's 32 qh bytes.
@@ -1022,7 +989,7 @@ static hipError_t gate_up_mfma_ts(const ExpertArgs& a, hipStream_t s) {
   const dim3 grid(a.I / 64, grid_tiles(a));
   switch (a.gate.fmt) {
     case HX_Q4_K: hx_launch(k_gate_up_q4k<1, 4, TS>, grid, dim3(256), 0, s, a); break;
-    case HX_Q8_0: hx_launch(k_gate_up_mfma<HX_Q8_0, TS>, grid, dim3(256), 0, s, a); break;
+    case HX_Q8_0: return launch_gate_up_q8(a, grid, s);
     case HX_Q6_K: hx_launch(k_gate_up_mfma<HX_Q6_K, TS>, grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
@@ -1042,7 +1009,7 @@ static hipError_t down_mfma_ts(const ExpertArgs& a, hipStream_t s) {
   const dim3 grid(a.H / 128, grid_tiles(a));
   switch (a.down.fmt) {
     case HX_Q4_K: hx_launch(k_down_mfma<HX_Q4_K, TS>, grid, dim3(256), 0, s, a); break;
-    case HX_Q8_0: hx_launch(k_down_mfma<HX_Q8_0, TS>, grid, dim3(256), 0, s, a); break;
+    case HX_Q8_0: return launch_down_q8(a, grid, s);
     case HX_Q6_K:
       if (a.I == DQ_K && (a.wpos || TS == HX_TILES_SHARED)) hx_launch(k_down_q6k<TS>, grid, dim3(256), 0, s, a);
       else hx_launch(k_down_mfma<HX_Q6_K, TS>, grid, dim3(256), 0, s, a);

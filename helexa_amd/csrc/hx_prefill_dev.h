@@ -30,12 +30,15 @@ HX_DEV bool get_tile(const ExpertArgs& a, int tile, int& e, int& p0, int& rows, 
     m = a.T;
     return true;
   }
-  if (tile >= a.counts[1]) return false;
-  m = a.tiles[4 * tile + 0];
-  e = a.tiles[4 * tile + 1];
-  p0 = a.tiles[4 * tile + 2];
-  rows = a.tiles[4 * tile + 3];
-  return !(TS == HX_TILES_ROUTED && e == a.E);
+  // the record read together with the tile count (one round trip, not two);
+  // the grid is rounded up past the list's last record
+  const int4 rec = *(const int4*)(a.tiles + 4 * min(tile, a.max_tiles - 1));
+  const int n = a.counts[1];
+  m = rec.x;
+  e = rec.y;
+  p0 = rec.z;
+  rows = rec.w;
+  return tile < n && !(TS == HX_TILES_ROUTED && e == a.E);
 }
 
 }  // namespace hx
