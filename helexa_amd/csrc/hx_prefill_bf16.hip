@@ -66,17 +66,23 @@ constexpr int BG_K = 128, BG_LD = BG_K + 8;
 constexpr int BG_OP = 68;   // pitch of the f32 tile of h (aliases the rows)
 
 template <int MT>
-HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const int* rowsrc, const uint8_t* G, const uint8_t* U,
-                            int rows, int p0, int n0) {
+HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const uint8_t* G, const uint8_t* U, int rows, int p0,
+                            int n0, bool sh) {
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, l16 = lane & 15, kq = lane >> 4;
   const int K = a.H, nk = K / BG_K;   // even
   // uniform bases and 32-bit lane offsets
   const uint8_t* bp[2] = {G + (int64_t)n0 * K * 2, U + (int64_t)n0 * K * 2};
   const uint32_t bo = (uint32_t)((16 * wave + l16) * K + 8 * kq) * 2;
   const int r0 = tid >> 4, seg = tid & 15;   // A piece i: row r0 + 16 i, elements 8 seg ..
-  const uint16_t* ap[MT];
+  // the rows' entries are read ahead of the first weight loads and used behind them
+  int src[MT];
 #pragma unroll
-  for (int i = 0; i < MT; i++) ap[i] = (const uint16_t*)a.x + (int64_t)rowsrc[r0 + 16 * i] * K + 8 * seg;
+  for (int i = 0; i < MT; i++) {
+    const int p = p0 + min(r0 + 16 * i, rows - 1);   // padding rows repeat the last row
+    src[i] = sh ? p : a.perm[p];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const uint16_t* ap[MT];
   u32x4_t ar[MT], b[2][2][4];
   auto load_a = [&](int kc) __attribute__((always_inline)) {
 #pragma unroll
@@ -97,8 +103,11 @@ HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const int* rowsrc
   for (int m = 0; m < 2; m++)
 #pragma unroll
     for (int i = 0; i < MT; i++) acc[m][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  load_a(0);
   load_b(0, ic<0>{});
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < MT; i++) ap[i] = (const uint16_t*)a.x + (int64_t)(sh ? src[i] - a.F : src[i] / a.k) * K + 8 * seg;
+  load_a(0);
   store_a(0);
   lds_barrier();
   auto step = [&](int kc, auto par, auto more) __attribute__((always_inline)) {
@@ -156,25 +165,19 @@ HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const int* rowsrc
 // grid (I / 64, tiles rounded up to 8), mapped by xcd_tile
 __global__ __launch_bounds__(256, 3) void k_gate_up_bf16(ExpertArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t As[2 * PM * BG_LD];
-  __shared__ int rowsrc[PM];
   static_assert(sizeof(float) * PM * BG_OP <= sizeof(As), "the tile of h fits the rows' LDS");
   int nt, tile, e, p0, rows, mc;
   xcd_tile(nt, tile);
   if (!get_tile<HX_TILES_ALL>(a, tile, e, p0, rows, mc)) return;
   const bool sh = e == a.E;
-  if (threadIdx.x < PM) {
-    const int p = p0 + min((int)threadIdx.x, rows - 1);   // padding rows repeat the last row
-    rowsrc[threadIdx.x] = sh ? p - a.F : a.perm[p] / a.k;
-  }
-  __syncthreads();
   const uint8_t* G = sh ? a.sgate.base : a.gate.mat(e);
   const uint8_t* U = sh ? a.sup.base : a.up.mat(e);
   const int n0 = nt * 64;
   switch ((rows + 15) >> 4) {   // uniform over the workgroup
-    case 1: bf_gate_up_main<1>(a, As, rowsrc, G, U, rows, p0, n0); break;
-    case 2: bf_gate_up_main<2>(a, As, rowsrc, G, U, rows, p0, n0); break;
-    case 3: bf_gate_up_main<3>(a, As, rowsrc, G, U, rows, p0, n0); break;
-    default: bf_gate_up_main<4>(a, As, rowsrc, G, U, rows, p0, n0); break;
+    case 1: bf_gate_up_main<1>(a, As, G, U, rows, p0, n0, sh); break;
+    case 2: bf_gate_up_main<2>(a, As, G, U, rows, p0, n0, sh); break;
+    case 3: bf_gate_up_main<3>(a, As, G, U, rows, p0, n0, sh); break;
+    default: bf_gate_up_main<4>(a, As, G, U, rows, p0, n0, sh); break;
   }
 }
 
@@ -189,7 +192,8 @@ constexpr int BD_K = 64, BD_PLANE = PM * BD_K, BD_STAGE = 3 * BD_PLANE;
 constexpr int BD_OP = 136;   // pitch of the bf16 output tile (aliases the rows)
 
 template <int MT>
-HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, const uint8_t* W, int K, int rows, int p0, int n0) {
+HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, float* rws, const uint8_t* W, int K, int rows, int p0, int n0,
+                         float rw) {
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, l16 = lane & 15, kq = lane >> 4;
   constexpr int NA = (MT + 1) / 2;   // rounds of 32 rows
   const int nc = K / 128;            // even
@@ -268,17 +272,18 @@ HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, const uint8_t* W, in
   step(nc - 2, ic<1>{}, ic<0>{}, ic<0>{});
   step(nc - 1, ic<0>{}, ic<1>{}, ic<1>{});
   step(nc - 1, ic<1>{}, ic<1>{}, ic<1>{});
+  if (tid < PM) rws[tid] = rw;
+  lds_barrier();
   uint16_t* ot = As;
 #pragma unroll
-  for (int i = 0; i < MT; i++)
+  for (int i = 0; i < MT; i++) {
+    const f32x4_t w = *(const f32x4_t*)(rws + 16 * i + 4 * kq);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int m = 16 * i + 4 * kq + q;
-      const float w = a.wpos[p0 + min(m, rows - 1)];
+    for (int q = 0; q < 4; q++)
 #pragma unroll
       for (int j = 0; j < 2; j++)
-        ot[m * BD_OP + 32 * wave + 16 * j + l16] = f32_to_bf16(w * acc[j][i][q]);
-    }
+        ot[(16 * i + 4 * kq + q) * BD_OP + 32 * wave + 16 * j + l16] = f32_to_bf16(w[q] * acc[j][i][q]);
+  }
   lds_barrier();
   const int c8 = 8 * (tid & 15);
 #pragma unroll
@@ -290,6 +295,7 @@ HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, const uint8_t* W, in
 // grid (H / 128, tiles rounded up to 8), mapped by xcd_tile
 __global__ __launch_bounds__(256, 3) void k_down_bf16(ExpertArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t As[2 * BD_STAGE];
+  __shared__ __attribute__((aligned(16))) float rws[PM];
   static_assert(PM * BD_OP <= 2 * BD_STAGE, "the output tile fits the rows' LDS");
   int nt, tile, e, p0, rows, mc;
   xcd_tile(nt, tile);
@@ -297,11 +303,13 @@ __global__ __launch_bounds__(256, 3) void k_down_bf16(ExpertArgs a) {
   const bool sh = e == a.E;
   const uint8_t* W = sh ? a.sdown.base : a.down.mat(e);
   const int K = sh ? a.Is : a.I, n0 = nt * 128;
+  // a row's routing weight, used by the epilogue
+  const float rw = threadIdx.x < PM ? a.wpos[p0 + min((int)threadIdx.x, rows - 1)] : 0.f;
   switch ((rows + 15) >> 4) {   // uniform over the workgroup
-    case 1: bf_down_main<1>(a, As, W, K, rows, p0, n0); break;
-    case 2: bf_down_main<2>(a, As, W, K, rows, p0, n0); break;
-    case 3: bf_down_main<3>(a, As, W, K, rows, p0, n0); break;
-    default: bf_down_main<4>(a, As, W, K, rows, p0, n0); break;
+    case 1: bf_down_main<1>(a, As, rws, W, K, rows, p0, n0, rw); break;
+    case 2: bf_down_main<2>(a, As, rws, W, K, rows, p0, n0, rw); break;
+    case 3: bf_down_main<3>(a, As, rws, W, K, rows, p0, n0, rw); break;
+    default: bf_down_main<4>(a, As, rws, W, K, rows, p0, n0, rw); break;
   }
 }
 
