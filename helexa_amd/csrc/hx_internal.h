@@ -234,6 +234,8 @@ hipError_t launch_down_mfma(const ExpertArgs& a, hipStream_t s);
 // Q8_0 weights; grid as the launches above
 hipError_t launch_gate_up_q8(const ExpertArgs& a, dim3 grid, hipStream_t s);
 hipError_t launch_down_q8(const ExpertArgs& a, dim3 grid, hipStream_t s);
+// the gate/up kernel writes the quantised arm's h as the f16 d q of its codes
+inline bool hq_in_gate_up(const ExpertArgs& a) { return a.gate.fmt == HX_Q8_0 && a.down.fmt == HX_Q8_0; }
 bool prefill_bf16_ok(const ExpertArgs& a);   // bf16 activations, bf16 experts: MFMA grouped GEMMs
 hipError_t launch_gate_up_bf16(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_down_bf16(const ExpertArgs& a, hipStream_t s);

@@ -733,7 +733,7 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
       tm_ext(m, SLOT_SH_GATE_UP, m->side);
       HX_HIP(launch_gate_up_mfma(sa, m->side));
       tm_ext_done(m, SLOT_SH_GATE_UP);
-      if (hq_shared) HX_HIP(launch_hq_fq(sa, (int)((T + HX_TILE_M - 1) / HX_TILE_M), m->side));
+      if (hq_shared && !hq_in_gate_up(sa)) HX_HIP(launch_hq_fq(sa, (int)((T + HX_TILE_M - 1) / HX_TILE_M), m->side));
       tm_ext(m, SLOT_SH_DOWN, m->side);
       HX_HIP(launch_down_mfma(sa, m->side));
       tm_ext_done(m, SLOT_SH_DOWN);
@@ -756,7 +756,7 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
       tm_ext(m, SLOT_GATE_UP, s);
       HX_HIP(launch_gate_up_mfma(p.ea, s));
       tm_ext_done(m, SLOT_GATE_UP);
-      HX_HIP(launch_hq_fq(p.ea, p.ea.max_tiles, s));
+      if (!hq_in_gate_up(p.ea)) HX_HIP(launch_hq_fq(p.ea, p.ea.max_tiles, s));
       tm_ext(m, SLOT_DOWN, s);
       HX_HIP(launch_down_mfma(p.ea, s));
       tm_ext_done(m, SLOT_DOWN);

@@ -32,6 +32,7 @@
 // l / 16 the 8 elements at Frag::pos(s, kq), which is where the lane's own 16
 // bytes of codes lie, instead of 32 s + 8 kq.
 #include "hx_prefill_dev.h"
+#include "hx_quant.h"
 #include <type_traits>
 
 namespace hx {
@@ -246,8 +247,11 @@ HX_DEV void pd_gate_up(const ExpertArgs& a, uint8_t* lds, const uint8_t* G, cons
 #pragma unroll
     for (int i = 0; i < MT; i++) ap[i] = X + (int64_t)(sh ? src[i] - a.F : src[i] / a.k) * K + 8 * (tid & 15);
   }, acc);
-  // h through LDS, out 16 bytes a thread: quantised arm f32 in natural order,
-  // else gate and up rounded to f16 and h in f16 in the swizzled order
+  // h through LDS, out 16 bytes a thread in the swizzled order: quantised arm
+  // the f16 d q of its codes where the down weights are Q8_0 too (the tile
+  // holds whole blocks of 32 columns; a kernel of its own with h in f32 out and
+  // in again took 5 to 8 us), f32 in natural order for k_hq_fq where they are
+  // not; else gate and up rounded to f16 and h in f16
   float* ot = (float*)lds;
 #pragma unroll
   for (int i = 0; i < MT; i++)
@@ -258,25 +262,26 @@ HX_DEV void pd_gate_up(const ExpertArgs& a, uint8_t* lds, const uint8_t* G, cons
       ot[(16 * i + 4 * kq + q) * OP + c] = siluf_(gr) * ur;
     }
   lds_barrier();
-  if (qa) {
-    constexpr int PR = NC / 4;   // threads a row
-    const int c4 = 4 * (tid % PR);
+  if (qa && a.down.fmt != HX_Q8_0) {
+    const int c4 = 4 * (tid & 15);
 #pragma unroll
-    for (int m = tid / PR; m < 16 * MT; m += 256 / PR)
+    for (int i = 0, m = tid >> 4; i < MT; i++, m += 16)
       if (m < rows) *(float4*)(a.hbuf + (int64_t)(p0 + m) * a.hstride + n0 + c4) = *(const float4*)(ot + m * OP + c4);
-  } else {
-    constexpr int PR = NC / 8;
-    const int c8 = 8 * (tid % PR);
-    for (int m = tid / PR; m < rows; m += 256 / PR) {
-      uint32_t o[4];
+    return;
+  }
+  const int c8 = 8 * (tid & 7);
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
-        const float4 v = *(const float4*)(ot + m * OP + c8 + 4 * j);
-        o[2 * j] = u32(h2_t{(_Float16)v.x, (_Float16)v.z});
-        o[2 * j + 1] = u32(h2_t{(_Float16)v.y, (_Float16)v.w});
-      }
-      *(u32x4_t*)(a.hbf + (int64_t)(p0 + m) * a.hstride + n0 + c8) = u32x4_t{o[0], o[1], o[2], o[3]};
-    }
+  for (int m = tid >> 3; m < 16 * MT; m += 32) {   // 16 MT rows: whole waves, which quant_group needs
+    const float4 u = *(const float4*)(ot + m * OP + c8), v = *(const float4*)(ot + m * OP + c8 + 4);
+    const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+    float q[8], d;
+    quant_group<HX_Q8_0>(x, q, d);
+    _Float16 h[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) h[j] = qa ? fq_f16(q[j], d) : (_Float16)x[j];
+    if (m < rows)
+      *(u32x4_t*)(a.hbf + (int64_t)(p0 + m) * a.hstride + n0 + c8) =
+          u32x4_t{u32(h2_t{h[0], h[2]}), u32(h2_t{h[1], h[3]}), u32(h2_t{h[4], h[6]}), u32(h2_t{h[5], h[7]})};
   }
 }
 

@@ -35,3 +35,14 @@ def test_q8_prefill_wide():
     from helexa_amd import synth
     b = Blk(2304, 4, 2, 4096, 0, True, synth.FMT_Q8_0, O.BF16, 702)
     b.check(b.x(40, seed=3), TOL_BF16, tag="q8 prefill H2304 I4096")
+
+
+@pytest.mark.parametrize("down", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T", [33, 160])
+def test_q8_gate_up_other_down(down, T):
+    """Q8_0 gate and up over k-quant down weights: h is quantised by its own
+    kernel there (blocks of 256), on both sides of the 64 rows"""
+    from helexa_amd import moe, synth
+    fmt = dict(synth.FMT_Q8_0, down=getattr(moe, down), sdown=getattr(moe, down))
+    b = Blk(512, 8, 4, 512, 512, True, fmt, O.BF16, 703)
+    b.check(b.x(T, seed=4), TOL_BF16, tag=f"q8 gate/up, {down} down T={T}")
