@@ -165,8 +165,9 @@ struct ExpertArgs {
   void* y;             // [T, H] act dtype
   int max_slots, max_tiles;
   const int32_t* plan;
-  // decoder residual folded into the decode down kernel: resid[t] becomes
-  // bf16(resid[t] + bf16(y[t])) in place of writing y (bf16 activations)
+  // decoder residual folded into the fast decode down kernel (bf16) and the
+  // prefill combine (f32 too, there a float pointer): resid[t] becomes
+  // bf16(resid[t] + bf16(y[t])) in place of writing y
   uint16_t* resid = nullptr;
   const float* wpos = nullptr;   // prefill: routing weight by permuted position (see DispatchArgs)
   // decode down partial sums [groups of HX_DOWN_ROWS rows of h][T][H] when the

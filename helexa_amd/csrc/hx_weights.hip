@@ -600,9 +600,53 @@ hipError_t launch_repack(int fmt, const void* src, int64_t count, int64_t rows, 
 
 // ---------------------------------------------------------------- RMSNorm
 // one block per token; f32 sum of squares (per-thread strided, then a fixed
-// tree), y = x * rsqrt(mean + eps) * (1 + w) rounded to the activation dtype
-__global__ __launch_bounds__(256) void k_rmsnorm(const void* x, bool bf, int64_t H, const float* w, float eps,
-                                                 void* y) {
+// tree), y = x * rsqrt(mean + eps) * (1 + w) rounded to the activation dtype.
+// Bound by latency: the token's (and the weight's) elements, NV a thread, are
+// loaded together and the token's kept in registers (element by element in a
+// loop, twice: 7.7 us for 27 tokens of 2048, 8.3 for 512, against 6.6 and 7).
+template <int NV>
+__global__ __launch_bounds__(256) void k_rmsnorm(const void* x, bool bf, int H, const float* w, float eps, void* y) {
+  __shared__ float red[128];
+  const int64_t t = blockIdx.x;
+  const int tid = threadIdx.x;
+  float v[NV], wv[NV];
+#pragma unroll
+  for (int j = 0; j < NV; j++) {   // elements past the end: 0, which adds nothing
+    const int i = tid + 256 * j;
+    v[j] = i < H ? ld_act(x, t * H + i, bf) : 0.f;
+    wv[j] = i < H ? w[i] : 0.f;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NV; j++) ss = __builtin_fmaf(v[j], v[j], ss);
+  // tree over 256: 128, 64 across waves, 32 .. 1 inside wave 0
+  if (tid >= 128) red[tid - 128] = ss;
+  __syncthreads();
+  if (tid < 128) ss += red[tid];
+  __syncthreads();
+  if (tid >= 64 && tid < 128) red[tid - 64] = ss;
+  __syncthreads();
+  if (tid < 64) {
+    ss += red[tid];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) ss += __shfl_down(ss, off, 64);
+    if (tid == 0) red[64] = ss;
+  }
+  __syncthreads();
+  const float inv = 1.0f / sqrtf(red[64] / (float)H + eps);
+#pragma unroll
+  for (int j = 0; j < NV; j++) {
+    const int i = tid + 256 * j;
+    if (i >= H) break;
+    const float o = v[j] * inv * (1.0f + wv[j]);
+    if (bf) ((uint16_t*)y)[t * H + i] = f32_to_bf16(o);
+    else ((float*)y)[t * H + i] = o;
+  }
+}
+
+// any H, element by element; same arithmetic
+__global__ __launch_bounds__(256) void k_rmsnorm_loop(const void* x, bool bf, int64_t H, const float* w, float eps,
+                                                      void* y) {
   __shared__ float red[256];
   const int64_t t = blockIdx.x;
   float ss = 0.f;
@@ -637,7 +681,12 @@ __global__ __launch_bounds__(256) void k_residual_add(void* x, const void* y, bo
 
 hipError_t launch_rmsnorm(const void* x, bool xbf, int64_t T, int64_t H, const float* w, float eps, void* y,
                           hipStream_t s) {
-  hipLaunchKernelGGL(k_rmsnorm, dim3((unsigned)T), dim3(256), 0, s, x, xbf, H, w, eps, y);
+  const dim3 g((unsigned)T);
+  // as many registers as the row needs; longer rows than 4096 loop
+  if (H <= 1024) hipLaunchKernelGGL(k_rmsnorm<4>, g, dim3(256), 0, s, x, xbf, (int)H, w, eps, y);
+  else if (H <= 2048) hipLaunchKernelGGL(k_rmsnorm<8>, g, dim3(256), 0, s, x, xbf, (int)H, w, eps, y);
+  else if (H <= 4096) hipLaunchKernelGGL(k_rmsnorm<16>, g, dim3(256), 0, s, x, xbf, (int)H, w, eps, y);
+  else hipLaunchKernelGGL(k_rmsnorm_loop, g, dim3(256), 0, s, x, xbf, H, w, eps, y);
   return hipGetLastError();
 }
 
