@@ -568,11 +568,14 @@ __global__ __launch_bounds__(64 * NW, 3) void k_gate_up_q4k(ExpertArgs a) {
 // f16 pattern (1024 + q, exact), (x - 1056) * (d * sc) with packed f16 ops.
 // Rows are scaled by their routing weight by position (the shared expert's
 // rows by its sigmoid gate) and written as bf16 to the per-assignment rows.
-constexpr int DQ_A = PM * 64 * 2;
+template <bool SM>   // SM: every tile has at most 32 rows
+struct Dq {
+  static constexpr int A = (SM ? 32 : PM) * 64 * 2;
+  static constexpr int STAGE = A + 128 * 64 + 128 * 8;
+};
 constexpr int DQ_BROW = 64;
 constexpr int DQ_B = 128 * DQ_BROW;
 constexpr int DQ_S = 128 * 8;
-constexpr int DQ_STAGE = DQ_A + DQ_B + DQ_S;
 constexpr int DQ_NST = 3;
 constexpr int DQ_K = 512;
 constexpr int DQ_NC = DQ_K / 64;
@@ -621,9 +624,10 @@ HX_DEV DqSrc dq_sources(const uint16_t* hbf, int hstride, int p0, int rows, cons
 
 // NA + 3 DMA instructions per wave and chunk: A round i moves rows
 // 32 i .. 32 i + 31 of h, so tiles of at most 32 rows (NA = 1) skip round 1
-template <int NA>
+template <int NA, bool SM>
 HX_DEV void dq_issue(uint32_t lds0, int st, const DqSrc& src, int c, int wave_u) {
-  const uint32_t sbase = lds0 + (uint32_t)(st * DQ_STAGE);
+  constexpr int DQ_A = Dq<SM>::A;
+  const uint32_t sbase = lds0 + (uint32_t)(st * Dq<SM>::STAGE);
   const int sb = c >> 2, n = (c >> 1) & 1;
   static_assert(128 % HX_Q6K_GROUP == 0, "a down tile's weight rows are whole groups of the stored layout");
   const int aoff = 2 * dq_col(c), qloff = c * (HX_Q6K_GROUP * 32), qhoff = (c >> 1) * (HX_Q6K_GROUP * 32);
@@ -641,9 +645,10 @@ HX_DEV uint32_t q6_pair(uint32_t lo4, uint32_t hi2, uint32_t knib, uint32_t kmag
 }
 
 // MT: 16-row M sub-tiles in use
-template <int P, int MT>   // chunk parity: quarters P and P + 2 of the half
+template <int P, int MT, bool SM>   // chunk parity: quarters P and P + 2 of the half
 HX_DEV void dq_compute(const lds_u8* st, const uint16_t* dl, int sb, f32x4_t (*acc)[4], int wave, int l16, int kq,
                        uint32_t knib, uint32_t kmagic, uint32_t k30) {
+  constexpr int DQ_A = Dq<SM>::A;
   const h2_t off = h2s(-1056.0f);
 #pragma unroll
   for (int j = 0; j < 2; j++) {
@@ -684,14 +689,15 @@ HX_DEV void dq_compute(const lds_u8* st, const uint16_t* dl, int sb, f32x4_t (*a
 // activation-fragment reads and A DMA rounds for the sub-tiles in use)
 // fa: the f16 arm (m > HX_QUANT_M): the products rounded to f16 (the
 // reference's forward_via_f16 output) before the routing weight
-template <int MT>
+template <int MT, bool SM>
 HX_DEV void dq_main(const ExpertArgs& a, uint8_t* ring, float* rws, const DqSrc& src, float rw, int rows, int p0,
                     int n0, int wave, int wave_u, int l16, int kq, bool fa) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8*)ring;
+  constexpr int DQ_STAGE = Dq<SM>::STAGE;
   const uint16_t* dl = (const uint16_t*)(ring + DQ_NST * DQ_STAGE);
   constexpr int NA = MT <= 2 ? 1 : 2;   // A rounds (32 rows each) the tile needs
 #pragma unroll
-  for (int c = 0; c < DQ_NST - 1; c++) dq_issue<NA>(lds0, c, src, c, wave_u);
+  for (int c = 0; c < DQ_NST - 1; c++) dq_issue<NA, SM>(lds0, c, src, c, wave_u);
   const uint32_t knib = __builtin_amdgcn_readfirstlane(0x000F000Fu), k30 = __builtin_amdgcn_readfirstlane(0x00300030u);
   uint32_t kmagic;
   asm("v_mov_b32 %0, 0x64006400" : "=v"(kmagic));
@@ -712,9 +718,9 @@ HX_DEV void dq_main(const ExpertArgs& a, uint8_t* ring, float* rws, const DqSrc&
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();   // chunk c is in LDS for every wave; stage (c - 1) % NST is free
-    if (c + DQ_NST - 1 < DQ_NC) dq_issue<NA>(lds0, (c + DQ_NST - 1) % DQ_NST, src, c + DQ_NST - 1, wave_u);
+    if (c + DQ_NST - 1 < DQ_NC) dq_issue<NA, SM>(lds0, (c + DQ_NST - 1) % DQ_NST, src, c + DQ_NST - 1, wave_u);
     const lds_u8* st = (const lds_u8*)ring + (c % DQ_NST) * DQ_STAGE;
-    dq_compute<decltype(par)::value, MT>(st, dl, c >> 2, acc, wave, l16, kq, knib, kmagic, k30);
+    dq_compute<decltype(par)::value, MT, SM>(st, dl, c >> 2, acc, wave, l16, kq, knib, kmagic, k30);
   };
   static_assert(DQ_NC % 2 == 0, "chunks come in pairs");
   for (int c = 0; c < DQ_NC; c += 2) {
@@ -752,8 +758,9 @@ HX_DEV void dq_main(const ExpertArgs& a, uint8_t* ring, float* rws, const DqSrc&
   }
 }
 
-template <int TS>
-__global__ __launch_bounds__(256, 3) void k_down_q6k(ExpertArgs a) {
+template <int TS, bool SM>
+__global__ __launch_bounds__(256, SM ? 4 : 3) void k_down_q6k(ExpertArgs a) {
+  constexpr int DQ_STAGE = Dq<SM>::STAGE;
   __shared__ __attribute__((aligned(16))) uint8_t ring[DQ_NST * DQ_STAGE + 128 * 4];
   __shared__ __attribute__((aligned(16))) float rws[PM];
   int nt, tile;
@@ -775,10 +782,13 @@ __global__ __launch_bounds__(256, 3) void k_down_q6k(ExpertArgs a) {
          lds0 + (uint32_t)(DQ_NST * DQ_STAGE + wave_u * 256));
   const DqSrc src = dq_sources(a.hbf, a.hstride, p0, rows, W, a.H, n0);
   switch ((rows + 15) >> 4) {   // uniform over the workgroup
-    case 1: dq_main<1>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
-    case 2: dq_main<2>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
-    case 3: dq_main<3>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
-    default: dq_main<4>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
+    case 1: dq_main<1, SM>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
+    case 2: dq_main<2, SM>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
+  }
+  if constexpr (!SM) switch ((rows + 15) >> 4) {
+    case 1: case 2: break;
+    case 3: dq_main<3, SM>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
+    default: dq_main<4, SM>(a, ring, rws, src, rw, rows, p0, n0, wave, wave_u, l16, kq, fa); break;
   }
 }
 
@@ -977,6 +987,14 @@ hipError_t launch_x_to_f16(const ExpertArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Up to this many tokens no expert call has more rows, so every tile is of one
+// or two 16-row sub-tiles, and the Q6_K down kernel that holds only those in LDS
+// (40 KB) runs four workgroups a CU instead of three: 12 tokens 25.1 -> 24.0 us,
+// 27 44.8 -> 41.2, 32 50.3 -> 47.0. (The same for the Q4_K gate/up kernel, whose
+// one-sub-tile tiles then lose their third ring stage: 12 tokens 29.4 -> 27.9 us,
+// but 16 36.4 -> 42.7 and 24 51.2 -> 53.1.)
+#define HX_SMALL_T 32
+
 // M tiles a launch's grid covers
 static int grid_tiles(const ExpertArgs& a) {
   const int n = a.tsel == HX_TILES_SHARED ? (a.T + PM - 1) / PM : a.max_tiles;
@@ -1011,7 +1029,8 @@ static hipError_t down_mfma_ts(const ExpertArgs& a, hipStream_t s) {
     case HX_Q4_K: hx_launch(k_down_mfma<HX_Q4_K, TS>, grid, dim3(256), 0, s, a); break;
     case HX_Q8_0: return launch_down_q8(a, grid, s);
     case HX_Q6_K:
-      if (a.I == DQ_K && (a.wpos || TS == HX_TILES_SHARED)) hx_launch(k_down_q6k<TS>, grid, dim3(256), 0, s, a);
+      if (a.I == DQ_K && TS == HX_TILES_ALL && a.T <= HX_SMALL_T) hx_launch(k_down_q6k<HX_TILES_ALL, true>, grid, dim3(256), 0, s, a);
+      else if (a.I == DQ_K) hx_launch(k_down_q6k<TS, false>, grid, dim3(256), 0, s, a);
       else hx_launch(k_down_mfma<HX_Q6_K, TS>, grid, dim3(256), 0, s, a);
       break;
     default: return hipErrorInvalidValue;
