@@ -294,6 +294,8 @@ __global__ __launch_bounds__(256) void k_router_dec(RouterArgs r, ExpertArgs a, 
       router_rows<true, RBF, TT, 1>(r, rb * 4 + wave, g * TT);
     return;
   }
+  if constexpr (FMT == HX_BF16) return;   // no records: its grid holds the router's workgroups only
+  else {
   // one workgroup per token: wave w quantises the token's elements 512 w ..
   // 512 w + 511 (each wave holds the whole row for the RMSNorm's sum)
   const int t = (int)blockIdx.x - nrb * ng;
@@ -302,6 +304,7 @@ __global__ __launch_bounds__(256) void k_router_dec(RouterArgs r, ExpertArgs a, 
     case 1: x_records<FMT, 1>(r, a, t, wave); break;
     case 2: x_records<FMT, 2>(r, a, t, wave); break;
     default: x_records<FMT, 4>(r, a, t, wave); break;
+  }
   }
 }
 
@@ -1263,6 +1266,135 @@ __global__ __launch_bounds__(64 * NW, 4) void k_down_pipe3(ExpertArgs a) {
   }
 }
 
+// ----------------------------------------------------------------------------
+// One token on bf16 experts (unquantised checkpoints; exact products, f32 sums,
+// h in f32): the same three kernels as one token on GGUF experts, for the same
+// shapes. The four generic kernels these replace take a launch for the routing
+// and read slots, entries and weights in dependent round trips: router 5.0,
+// routing 7.0, gate/up 12.0, down 9.2 us; this: router 3.8, gate/up 11.3, down
+// 5.4 (46 and 23 MB of weights, 80B-A3B layer).
+//
+// Rows are read 512 elements a load: lane l holds elements 512 i + 8 l .. + 7 of
+// load i, so every load is one contiguous kilobyte.
+// ----------------------------------------------------------------------------
+// sum over this lane's 8 elements of w x, onto s
+HX_DEV float dot_bf8(u32x4v w, const float (&x)[8], float s) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    s = __builtin_fmaf(__uint_as_float(w[j] << 16), x[2 * j], s);
+    s = __builtin_fmaf(__uint_as_float(w[j] & 0xffff0000u), x[2 * j + 1], s);
+  }
+  return s;
+}
+
+// as k_gate_up_dec1, which see; H = 2048
+template <int EPL, int KR>
+__global__ __launch_bounds__(256) void k_gate_up_dec1_bf16(RouterArgs r, ExpertArgs a) {
+  constexpr int NL = 4;   // loads of a row
+  static_assert(KR < 16, "the rank-r sums and the shared one fit 16 values");
+  __shared__ float sums[4][16];
+  const int wave = threadIdx.x >> 6, lane = lane_id();
+  const int mat = wave & 1;                       // 0: gate, 1: up
+  const int row = blockIdx.x * 2 + (wave >> 1);   // row of I (and of the shared expert's Is)
+  const int K = a.H;
+  float lv[EPL];
+  route_logits_load<EPL>(r.logits, r.E, lv);
+  int sgi = r.has_shared ? r.E : 0;
+  asm volatile("" : "+v"(sgi));
+  const float sg = r.logits[sgi];
+  u32x4v xr[NL];
+#pragma unroll
+  for (int i = 0; i < NL; i++) xr[i] = *(const u32x4v*)((const uint16_t*)a.x + 512 * i + 8 * lane);
+  const bool shrow = a.Is > 0 && row < a.Is, rrow = row < a.I;
+  auto load_row = [&](const uint8_t* m, int rw, u32x4v (&v)[NL]) __attribute__((always_inline)) {
+    const uint16_t* p = (const uint16_t*)m + (int64_t)rw * K + 8 * lane;
+#pragma unroll
+    for (int i = 0; i < NL; i++) v[i] = *(const u32x4v*)(p + 512 * i);
+  };
+  const bool hs = a.Is > 0;   // without a shared expert, read routed matrix 0
+  u32x4v rsh[NL], raw[KR][NL];
+  load_row(hs ? (mat ? a.sup.base : a.sgate.base) : (mat ? a.up.mat(0) : a.gate.mat(0)), shrow ? row : 0, rsh);
+  __builtin_amdgcn_sched_barrier(0);
+  int my_e, e0 = 0;
+  float my_w;
+  route_token_core_hook<EPL, KR, 1>(lv, r.E, r.norm, my_e, my_w, [&](int j, int e) __attribute__((always_inline)) {
+    if (j < 0) {
+      e0 = e >= 0 ? e : 0;
+      load_row(mat ? a.up.mat(e0) : a.gate.mat(e0), rrow ? row : 0, raw[0]);
+    } else if (j >= 1 || e != e0) {
+      load_row(mat ? a.up.mat(e) : a.gate.mat(e), rrow ? row : 0, raw[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  int pos = 0;   // dispatch position of rank `lane`
+#pragma unroll
+  for (int j = 0; j < KR; j++) pos += __builtin_amdgcn_readlane(my_e, j) < my_e;
+  if (blockIdx.x == 0 && wave == 0)
+    publish_one_token(r.d, r.topk_w, r.sgw, my_e, my_w, pos, r.has_shared ? sigmoidf_(sg_late(sg)) : 0.0f);
+  float x[NL][8];
+#pragma unroll
+  for (int i = 0; i < NL; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      x[i][2 * j] = __uint_as_float(xr[i][j] << 16);
+      x[i][2 * j + 1] = __uint_as_float(xr[i][j] & 0xffff0000u);
+    }
+  float v[16];
+#pragma unroll
+  for (int j = 0; j < 16; j++) v[j] = 0.f;
+#pragma unroll
+  for (int i = 0; i < NL; i++) v[KR] = dot_bf8(rsh[i], x[i], v[KR]);
+  if (!hs) v[KR] = 0.f;
+#pragma unroll
+  for (int j = 0; j < KR; j++)
+#pragma unroll
+    for (int i = 0; i < NL; i++) v[j] = dot_bf8(raw[j][i], x[i], v[j]);
+  rs_vals64<16>(v);   // lane l: value l / 4
+  if ((lane & 3) == 0) sums[wave][lane >> 2] = v[0];
+  __syncthreads();
+  if (mat == 0 && lane <= KR) {
+    const float h = siluf_(sums[wave][lane]) * sums[wave + 1][lane];
+    if (lane < KR && rrow) a.hbuf[(int64_t)pos * a.hstride + row] = h;
+    if (lane == KR && shrow) a.hbuf[(int64_t)a.F * a.hstride + row] = h;
+  }
+}
+
+// I = 512; workgroup: 8 output rows, wave w the row w of h (at most 12), whose
+// weight, expert and 512 values it reads itself; contributions summed in row
+// order
+__global__ __launch_bounds__(64 * 12) void k_down_one_bf16(ExpertArgs a) {
+  constexpr int NO = 8, ROWS = 12;
+  __shared__ float contrib[ROWS][NO];
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
+  const int nh = a.F + (a.Is > 0 ? 1 : 0);   // rows of h in use (<= ROWS)
+  const int n0 = blockIdx.x * NO, n_out = n0 + (int)threadIdx.x;
+  // the residual this thread adds in the epilogue, loaded first by every thread (in bounds)
+  const uint16_t rx = a.resid ? a.resid[min(n_out, a.H - 1)] : 0;
+  const int hr = min(w, nh - 1);
+  const int tok0 = plan_rows_at(a), NH = a.F + 1;
+  const float wt = __int_as_float(a.plan[tok0 + NH + hr]);
+  const int e = a.plan[tok0 + 2 * NH + hr];
+  const float4* hp = (const float4*)(a.hbuf + (int64_t)hr * a.hstride + 8 * lane);
+  const float4 h0 = hp[0], h1 = hp[1];
+  const uint16_t* W = (const uint16_t*)(e == a.E ? a.sdown.base : a.down.mat(e)) + 8 * lane;
+  u32x4v raw[NO];
+#pragma unroll
+  for (int i = 0; i < NO; i++) raw[i] = *(const u32x4v*)(W + (int64_t)min(n0 + i, a.H - 1) * 512);
+  const float h[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+  float v[NO];
+#pragma unroll
+  for (int i = 0; i < NO; i++) v[i] = dot_bf8(raw[i], h, 0.f);
+  rs_vals64<NO>(v);   // lane l: value l / 8
+  if ((lane & 7) == 0) contrib[w][lane >> 3] = wt * v[0];
+  __syncthreads();
+  if (threadIdx.x < NO && n_out < a.H) {
+    float y = 0.f;
+    for (int j = 0; j < nh; j++) y += contrib[j][threadIdx.x];
+    if (a.resid) a.resid[n_out] = f32_to_bf16(resid_f32(rx) + bf16_to_f32(f32_to_bf16(y)));
+    else ((uint16_t*)a.y)[n_out] = f32_to_bf16(y);
+  }
+}
+
 // sum of the down kernel's per-group partials, in group order, for T tokens
 __global__ __launch_bounds__(256) void k_down_reduce(ExpertArgs a, int groups) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -1289,6 +1421,12 @@ bool decode_fast_ok(const ExpertArgs& a) {
   return a.xbf && same && ok(a.gate.fmt, a.H) && ok(a.down.fmt, Kd) && (a.Is == 0 || a.Is == a.I);
 }
 
+// one token on bf16 experts: the shapes of the overlapped kernel (below)
+bool decode_bf16_ok(const ExpertArgs& a) {
+  return a.xbf && a.T == 1 && a.gate.fmt == HX_BF16 && a.down.fmt == HX_BF16 && a.H == 2048 && a.I == 512 &&
+         (a.Is == 0 || a.Is == 512) && a.k == 10 && a.E > 256 && a.E <= 512;
+}
+
 template <int FMT>
 static hipError_t router_dec_fmt(const RouterArgs& r, const ExpertArgs& a, bool rbf, hipStream_t s) {
   // One router row a wave, the tokens in pairs: each pair's router
@@ -1300,10 +1438,15 @@ static hipError_t router_dec_fmt(const RouterArgs& r, const ExpertArgs& a, bool 
   // each).
 #define RD(RB, TT)                                                                          \
   {                                                                                         \
-    const int nrb = (r.E1 + 3) / 4, ng = (a.T + TT - 1) / TT, ncb = a.T;                    \
+    const int nrb = (r.E1 + 3) / 4, ng = (a.T + TT - 1) / TT, ncb = FMT == HX_BF16 ? 0 : a.T;                    \
     hx_launch(k_router_dec<FMT, RB, TT>, dim3(nrb * ng + ncb), dim3(256), 0, s, r, a, nrb); \
   }
-#define RD_T(RB) { if (r.T <= 1) RD(RB, 1) else RD(RB, 2) }
+#define RD_T(RB)                                           \
+  {                                                        \
+    if constexpr (FMT == HX_BF16) RD(RB, 1) /* one token */ \
+    else if (r.T <= 1) RD(RB, 1)                           \
+    else RD(RB, 2)                                         \
+  }
   if (rbf) RD_T(true) else RD_T(false)
 #undef RD_T
 #undef RD
@@ -1405,6 +1548,7 @@ hipError_t launch_router_dec(const RouterArgs& r, const ExpertArgs& a, bool rbf,
     case HX_Q8_0: return router_dec_fmt<HX_Q8_0>(r, a, rbf, s);
     case HX_Q4_K: return router_dec_fmt<HX_Q4_K>(r, a, rbf, s);
     case HX_Q6_K: return router_dec_fmt<HX_Q6_K>(r, a, rbf, s);
+    case HX_BF16: return router_dec_fmt<HX_BF16>(r, a, rbf, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1423,6 +1567,9 @@ hipError_t launch_gate_up_dec(const RouterArgs& r, const ExpertArgs& a, hipStrea
       case HX_Q8_0: return gate_up_dec1_fmt<HX_Q8_0>(r, a, s);
       case HX_Q4_K: return gate_up_dec1_fmt<HX_Q4_K>(r, a, s);
       case HX_Q6_K: return gate_up_dec1_fmt<HX_Q6_K>(r, a, s);
+      case HX_BF16:
+        hx_launch(k_gate_up_dec1_bf16<8, 10>, dim3((a.I + 1) / 2), dim3(256), 0, s, r, a);
+        return hipGetLastError();
       default: break;
     }
   }
@@ -1448,6 +1595,10 @@ hipError_t launch_down_dec(const ExpertArgs& a, hipStream_t s) {
     case HX_Q8_0: return down_dec_fmt<HX_Q8_0>(a, s);
     case HX_Q4_K: return down_dec_fmt<HX_Q4_K>(a, s);
     case HX_Q6_K: return down_dec_fmt<HX_Q6_K>(a, s);
+    case HX_BF16:
+      if (!decode_bf16_ok(a) || a.hstride != 512) return hipErrorInvalidValue;
+      hx_launch(k_down_one_bf16, dim3((a.H + 7) / 8), dim3(64 * 12), 0, s, a);
+      return hipGetLastError();
     default: return hipErrorInvalidValue;
   }
 }

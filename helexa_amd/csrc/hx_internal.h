@@ -221,6 +221,7 @@ hipError_t launch_row_norms(const void* R, int E1, int H, float* out, hipStream_
 
 // decode (T <= HX_DECODE_MAX_T)
 bool decode_fast_ok(const ExpertArgs& a);   // bf16 activations, GGUF weights: f16 dot2 kernels
+bool decode_bf16_ok(const ExpertArgs& a);   // one token, bf16 experts: the same kernels' bf16 forms
 hipError_t launch_router_dec(const RouterArgs& r, const ExpertArgs& a, bool rbf, hipStream_t s);  // router + shared gate/up
 hipError_t launch_gate_up_dec(const RouterArgs& r, const ExpertArgs& a, hipStream_t s);   // T == 1: routes in its prologue
 hipError_t launch_gate_up_plan(const ExpertArgs& a, hipStream_t s);   // T > 1: reads the published plan

@@ -636,12 +636,12 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
   Plan p;
   make_plan(m, x, T, y, (uint8_t*)ws, L, bias, p);
   const bool decode = T <= HX_DECODE_MAX_T;
-  const bool fast = decode && decode_fast_ok(p.ea);
+  const bool fast = decode && (decode_fast_ok(p.ea) || decode_bf16_ok(p.ea));
   p.ra.d.plan_only = fast;   // the fast kernels read the plan only
   const bool bf = m->cfg.act_dtype == HX_BF16;
   const int H = m->cfg.hidden_size;
   uint16_t* xn = (uint16_t*)((uint8_t*)ws + L.xn);
-  if (fz && fast && H <= 8 * 256) {
+  if (fz && fast && gguf_fmt(m->gate.fmt) && H <= 8 * 256) {
     // RMSNorm inside the router kernel (the router waves and the token-record
     // waves normalise each token with the same arithmetic, so both see the
     // same bits), residual inside the down kernel
