@@ -56,9 +56,12 @@ template <int FMT, int LPR, int CPL, int NTOK, int NRG>
 __global__ __launch_bounds__(256) void k_gate_up(ExpertArgs a) {
   using CK = Chunk<FMT>;
   constexpr int CH = CK::CH, RG = 64 / LPR, NS = CK::NSUM > 0 ? CK::NSUM : 1;
+  // the slot's record read together with the slot count (u < max_slots, so the
+  // record exists), and its first tokens' entries together with the weights:
+  // one round trip less each
   const int u = blockIdx.y;
-  if (u >= a.counts[0]) return;
   const int e = a.slots[3 * u], start = a.slots[3 * u + 1], count = a.slots[3 * u + 2];
+  if (u >= a.counts[0]) return;
   const bool sh = e == a.E;
   const uint8_t* G = sh ? a.sgate.base : a.gate.mat(e);
   const uint8_t* U = sh ? a.sup.base : a.up.mat(e);
@@ -72,7 +75,11 @@ __global__ __launch_bounds__(256) void k_gate_up(ExpertArgs a) {
   // come as the f32 d q of their codes (k_xq_f32)
   const bool qa = a.xq32 && count <= HX_QUANT_M;
 
-  // weights first: every load of the wave is in flight before any math
+  // the entries of the first tokens (scalar loads), then the weights: every load
+  // of the wave is in flight before any math
+  int ent[NTOK];
+#pragma unroll
+  for (int tok = 0; tok < NTOK; tok++) ent[tok] = sh ? min(tok, count - 1) : a.perm[start + min(tok, count - 1)];
   typename CK::Raw rgt[NRG][CPL], rup[NRG][CPL];
 #pragma unroll
   for (int g = 0; g < NRG; g++) {
@@ -92,7 +99,7 @@ __global__ __launch_bounds__(256) void k_gate_up(ExpertArgs a) {
 #pragma unroll
     for (int tok = 0; tok < NTOK; tok++) {
       const int j = tg + tok < count ? tg + tok : count - 1;
-      const int t = sh ? j : a.perm[start + j] / a.k;
+      const int t = sh ? j : (tg == 0 ? ent[tok] : a.perm[start + j]) / a.k;
       hrow[tok] = sh ? a.F + j : start + j;
       const bool xb = a.xbf && !qa;
       const void* xr = qa ? (const void*)(a.xq32 + (int64_t)t * K)
@@ -135,71 +142,70 @@ __global__ __launch_bounds__(256) void k_gate_up(ExpertArgs a) {
 
 // ----------------------------------------------------------------------------
 // decode down projection + combine. Block = RG output rows (one wave-row-group);
-// its 4 waves split the slots; contrib[u][t][r] collects w * (down_e row . h)
-// in LDS and the final sum runs over u in slot order (experts ascending, then
-// the shared expert), as moe.rs:178-194 does.
+// its 4 waves split the rows of h in dispatch order (the routed rows by expert,
+// then the shared expert's), whose token, weight and expert come from the decode
+// plan; contrib[hr][r] collects weight * (down_e row . h) in LDS and each token's
+// output sums its rows in that order (experts ascending, then the shared
+// expert), as moe.rs:178-194 does. Bound by latency at the sizes that come here:
+// plan, then weights and rows of h together (by slot list, permutation and
+// routing weights in turn, the rows of h behind the weights: 8.0 us for 4 tokens
+// of the 256-wide f32 block, 7.4 so; 54 -> 47 us a forward of 2 bf16 tokens).
 // ----------------------------------------------------------------------------
 template <int FMT, int LPR, int CPL, int SPW>
 __global__ __launch_bounds__(256) void k_down_combine(ExpertArgs a) {
   using CK = Chunk<FMT>;
   constexpr int CH = CK::CH, RG = 64 / LPR, NS = CK::NSUM > 0 ? CK::NSUM : 1;
+  constexpr bool HPRE = CPL * CH <= 16;   // rows of h short enough to be held beside the weights
   extern __shared__ float contrib[];
-  const int nslots = a.counts[0], T = a.T;
-  const int lane = lane_id(), wave = threadIdx.x >> 6, rg = lane / LPR, ll = lane % LPR;
+  const int T = a.T, NH = a.F + T, nr = a.F + (a.Is > 0 ? T : 0);   // plan stride; rows of h in use
+  int* stok = (int*)(contrib + nr * RG);
+  const int32_t* plan = a.plan + 4 + 4 * a.max_slots;   // tokens, weights, experts of the rows
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int rg = lane / LPR, ll = lane % LPR;
   const int n0 = blockIdx.x * RG, row = n0 + rg;
-  for (int i = threadIdx.x; i < nslots * T * RG; i += 256) contrib[i] = 0.f;
-  __syncthreads();
-  for (int ub = wave; ub < nslots; ub += 4 * SPW) {
+  for (int i = threadIdx.x; i < nr; i += 256) stok[i] = plan[i];
+  for (int hb = wave; hb < nr; hb += 4 * SPW) {
     typename CK::Raw raw[SPW][CPL];
+    float wgt[SPW], hv[SPW][HPRE ? CPL * CH : 1];
+    int Ks[SPW];
 #pragma unroll
     for (int s = 0; s < SPW; s++) {
-      const int u = ub + 4 * s;
-      if (u < nslots) {
-        const int e = a.slots[3 * u];
-        const bool sh = e == a.E;
-        const uint8_t* W = sh ? a.sdown.base : a.down.mat(e);
-        const int K = sh ? a.Is : a.I;
+      const int hr = min(hb + 4 * s, nr - 1), e = plan[2 * NH + hr];
+      const bool sh = e == a.E;
+      wgt[s] = __int_as_float(plan[NH + hr]);
+      Ks[s] = sh ? a.Is : a.I;
+      const uint8_t* W = sh ? a.sdown.base : a.down.mat(e);
 #pragma unroll
-        for (int ci = 0; ci < CPL; ci++) {
-          const int c = ll + LPR * ci;
-          if (row < a.H && c < K / CH) CK::load(W, a.H, K, row, c, raw[s][ci]);
+      for (int ci = 0; ci < CPL; ci++) {
+        const int c = ll + LPR * ci;
+        if (hb + 4 * s < nr && row < a.H && c < Ks[s] / CH) {
+          CK::load(W, a.H, Ks[s], row, c, raw[s][ci]);
+          if constexpr (HPRE) load_chunk_x<FMT>(a.hbuf + (int64_t)hr * a.hstride, false, c, hv[s] + CH * ci);
         }
       }
     }
 #pragma unroll
     for (int s = 0; s < SPW; s++) {
-      const int u = ub + 4 * s;
-      if (u >= nslots) break;
-      const int e = a.slots[3 * u], start = a.slots[3 * u + 1], count = a.slots[3 * u + 2];
-      const bool sh = e == a.E;
-      const int K = sh ? a.Is : a.I;
-      for (int j = 0; j < count; j++) {
-        int t, hrow;
-        float wgt;
-        if (sh) {
-          t = j;
-          hrow = a.F + j;
-          wgt = a.sgw[j];
-        } else {
-          const int f = a.perm[start + j];
-          t = f / a.k;
-          hrow = start + j;
-          wgt = a.topk_w[f];
-        }
-        float p = 0.f;
+      const int hr = hb + 4 * s;
+      if (hr >= nr) break;
+      float p = 0.f;
 #pragma unroll
-        for (int ci = 0; ci < CPL; ci++) {
-          const int c = ll + LPR * ci;
-          if (c < K / CH) {
-            float xv[CH], xs[NS];
-            load_chunk_x<FMT>(a.hbuf + (int64_t)hrow * a.hstride, false, c, xv);
-            CK::sums(xv, xs);
-            p += CK::dot(raw[s][ci], xv, xs);
+      for (int ci = 0; ci < CPL; ci++) {
+        const int c = ll + LPR * ci;
+        if (row < a.H && c < Ks[s] / CH) {
+          float xv[CH], xs[NS];
+          if constexpr (HPRE) {
+#pragma unroll
+            for (int j = 0; j < CH; j++) xv[j] = hv[s][CH * ci + j];
+          } else {
+            load_chunk_x<FMT>(a.hbuf + (int64_t)hr * a.hstride, false, c, xv);
           }
+          CK::sums(xv, xs);
+          p += CK::dot(raw[s][ci], xv, xs);
         }
-        p = wave_sum<LPR>(p);
-        if (ll == 0 && row < a.H) contrib[((int64_t)u * T + t) * RG + rg] = wgt * p;
       }
+      p = wave_sum<LPR>(p);
+      if (ll == 0) contrib[hr * RG + rg] = wgt[s] * p;
     }
   }
   __syncthreads();
@@ -207,7 +213,7 @@ __global__ __launch_bounds__(256) void k_down_combine(ExpertArgs a) {
     const int t = i / RG, r = i % RG;
     if (n0 + r >= a.H) continue;
     float y = 0.f;
-    for (int u = 0; u < nslots; u++) y += contrib[((int64_t)u * T + t) * RG + r];
+    for (int hr = 0; hr < nr; hr++) y += stok[hr] == t ? contrib[hr * RG + r] : 0.f;
     const int64_t o = (int64_t)t * a.H + n0 + r;
     if (a.xbf) ((uint16_t*)a.y)[o] = f32_to_bf16(y);
     else ((float*)a.y)[o] = y;
@@ -418,7 +424,7 @@ static hipError_t down_combine_fmt(const ExpertArgs& a, hipStream_t s) {
 #define DC(LPR, CPL)                                                                            \
   {                                                                                             \
     constexpr int RG = 64 / LPR;                                                                \
-    size_t lds = (size_t)a.max_slots * a.T * RG * sizeof(float);                                \
+    size_t lds = (size_t)(a.F + a.T) * (RG + 1) * sizeof(float);                                \
     hipLaunchKernelGGL((k_down_combine<FMT, LPR, CPL, 4>), dim3((a.H + RG - 1) / RG), dim3(256), \
                        lds, s, a);                                                              \
   }
