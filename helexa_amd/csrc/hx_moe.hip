@@ -653,8 +653,9 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
   } else if (fz) {
     HX_HIP(launch_rmsnorm(fz->x, bf, T, H, fz->norm_w, fz->eps, xn, s));
     p.ra.x = p.ea.x = xn;
-    // the down kernel (fast decode) or the combine (prefill) adds the residual
-    if (fast || !decode) p.ea.resid = (uint16_t*)fz->x;
+    // the down kernel (fast decode) or the combine (prefill, 16 bytes of the
+    // stream a thread) adds the residual
+    if (fast || (!decode && ((uintptr_t)fz->x & 15) == 0)) p.ea.resid = (uint16_t*)fz->x;
   }
   if (fast) {
     // router + shared gate/up; routed gate/up (one token: routing in its

@@ -26,3 +26,18 @@ def test_decoder_prefill(H, fmt, act, T):
     ref = x.float().cpu().numpy() + b.ref(x_np(n))
     got = b.block.decoder_mlp_(x.clone(), w, 1e-6).float().cpu().numpy()
     assert rel_err(got, ref) <= (TOL_BF16 if act == O.BF16 else TOL_F32)
+
+
+@pytest.mark.parametrize("act,offset", [(O.BF16, 1), (O.BF16, 4), (O.F32, 1)])
+def test_residual_stream_at_any_element(act, offset):
+    """a stream that does not start on 16 bytes: same bits as one that does"""
+    import torch
+    from helexa_amd import synth
+    H, T = 768, 21
+    b = Blk(H, 8, 2, 256, 256, True, synth.FMT_Q8_0 if act == O.BF16 else synth.FMT_F32, act, 41)
+    x = b.x(T, seed=3)
+    w = torch.linspace(-0.5, 0.5, H, device="cuda")
+    buf = torch.empty(T * H + 8, dtype=x.dtype, device="cuda")
+    off = buf[offset:offset + T * H].view(T, H).copy_(x)
+    assert off.data_ptr() % 16 != 0
+    assert torch.equal(b.block.decoder_mlp_(off, w, 1e-6), b.block.decoder_mlp_(x.clone(), w, 1e-6))
