@@ -159,7 +159,7 @@ struct ExpertArgs {
   uint32_t* hrec;      // [(F+T)][I / 32][HX_XCV_WORDS] decode: the rows of h as chunk records
                        // (the down weights' vec_dot type)
   void* obuf;          // [(F+T), H] weighted expert outputs (prefill): bf16 for bf16
-                       // activations, f32 for f32 ones
+                       // activations, f32 for f32 ones and for few_bf16_ok
   const int32_t* inv;
   const int32_t* topk_idx;
   void* y;             // [T, H] act dtype
@@ -239,6 +239,10 @@ hipError_t launch_down_q8(const ExpertArgs& a, dim3 grid, hipStream_t s);
 // the gate/up kernel writes the quantised arm's h as the f16 d q of its codes
 inline bool hq_in_gate_up(const ExpertArgs& a) { return a.gate.fmt == HX_Q8_0 && a.down.fmt == HX_Q8_0; }
 bool prefill_bf16_ok(const ExpertArgs& a);   // bf16 activations, bf16 experts: MFMA grouped GEMMs
+// 5 .. HX_DECODE_MAX_T tokens, bf16 experts: the same GEMMs over the decode
+// plan's slots, f32 rows and a combine of their own
+bool few_bf16_ok(const ExpertArgs& a);
+hipError_t launch_combine_few(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_gate_up_bf16(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_down_bf16(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_gate_up_prefill(const ExpertArgs& a, hipStream_t s);

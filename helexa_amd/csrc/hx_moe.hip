@@ -20,6 +20,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "hx_moe.h"
@@ -179,7 +180,11 @@ static WsLayout ws_layout(const hx_moe* m, int64_t T) {
   L.hbuf = take(sizeof(float) * (F + T) * L.hstride);
   L.hbf = take(sizeof(uint16_t) * (F + T) * L.hstride);
   const size_t act = m->cfg.act_dtype == HX_BF16 ? 2 : 4;
-  L.obuf = decode ? 0 : take(act * (F + T) * H);
+  ExpertArgs sa = shape_args(m);
+  sa.T = (int)T;
+  sa.k = (int)k;
+  const bool few = few_bf16_ok(sa);
+  L.obuf = few ? take(sizeof(float) * (F + T) * H) : decode ? 0 : take(act * (F + T) * H);
   L.xh = decode ? 0 : take(sizeof(uint16_t) * T * H);
   const bool generic = generic_path(m, T);
   // the MFMA path's xq lives in the routed rows of the weighted-rows buffer,
@@ -191,11 +196,11 @@ static WsLayout ws_layout(const hx_moe* m, int64_t T) {
     L.xq = at + need <= act * F * H ? L.obuf + at : take(need);
   }
   L.xq32 = generic && gguf_fmt(m->gate.fmt) ? take(sizeof(float) * T * H) : 0;
-  L.xcv = decode ? take(sizeof(uint32_t) * (size_t)T * (H / 32) * HX_XCV_WORDS) : 0;
-  L.hrec = decode ? take(sizeof(uint32_t) * (size_t)(F + T) * ((I > Is ? I : Is) / 32) * HX_XCV_WORDS) : 0;
+  L.xcv = decode && !few ? take(sizeof(uint32_t) * (size_t)T * (H / 32) * HX_XCV_WORDS) : 0;
+  L.hrec = decode && !few ? take(sizeof(uint32_t) * (size_t)(F + T) * ((I > Is ? I : Is) / 32) * HX_XCV_WORDS) : 0;
   L.xn = take(act * T * H);
   L.ym = take(act * T * H);
-  L.dpart = decode ? take(sizeof(float) * (size_t)down_groups((int)F, (int)T) * T * H) : 0;
+  L.dpart = decode && !few ? take(sizeof(float) * (size_t)down_groups((int)F, (int)T) * T * H) : 0;
   L.wpos = decode ? 0 : take(sizeof(float) * (F + T));
   L.total = o;
   return L;
@@ -405,7 +410,10 @@ extern "C" int hx_moe_create(const hx_moe_config* cfg, const hx_moe_weights* w, 
 
 extern "C" int hx_moe_workspace_size(const hx_moe* m, int64_t n_tokens, size_t* bytes) {
   if (!m || !bytes || n_tokens < 0) return fail(HX_ERR_INVALID_ARGUMENT, "bad argument");
-  *bytes = ws_layout(m, n_tokens).total;
+  // never less than a call of fewer tokens takes: up to HX_DECODE_MAX_T tokens on
+  // bf16 experts hold their weighted rows in f32, larger calls in bf16
+  const int64_t few = n_tokens < HX_DECODE_MAX_T ? n_tokens : HX_DECODE_MAX_T;
+  *bytes = std::max(ws_layout(m, n_tokens).total, ws_layout(m, few).total);
   return HX_OK;
 }
 
@@ -517,7 +525,8 @@ static void make_plan(hx_moe* m, const void* x, int64_t T, void* y, uint8_t* ws,
   a.max_tiles = L.max_tiles;
   a.plan = d.plan;
   a.dpart = L.dpart ? (float*)(ws + L.dpart) : nullptr;
-  a.wpos = d.wpos;
+  // the plan holds the routing weights by position too
+  a.wpos = few_bf16_ok(a) ? (const float*)(d.plan + 4 + 4 * L.max_slots + F + T) : d.wpos;
 }
 
 namespace hx {
@@ -641,6 +650,7 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
   const bool bf = m->cfg.act_dtype == HX_BF16;
   const int H = m->cfg.hidden_size;
   uint16_t* xn = (uint16_t*)((uint8_t*)ws + L.xn);
+  const bool few = decode && !fast && few_bf16_ok(p.ea);
   if (fz && fast && gguf_fmt(m->gate.fmt) && H <= 8 * 256) {
     // RMSNorm inside the router kernel (the router waves and the token-record
     // waves normalise each token with the same arithmetic, so both see the
@@ -653,9 +663,9 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
   } else if (fz) {
     HX_HIP(launch_rmsnorm(fz->x, bf, T, H, fz->norm_w, fz->eps, xn, s));
     p.ra.x = p.ea.x = xn;
-    // the down kernel (fast decode) or the combine (prefill, 16 bytes of the
+    // the down kernel (fast decode) or the combine (up to 16 bytes of the
     // stream a thread) adds the residual
-    if (fast || (!decode && ((uintptr_t)fz->x & 15) == 0)) p.ea.resid = (uint16_t*)fz->x;
+    if (fast || ((!decode || few) && ((uintptr_t)fz->x & 15) == 0)) p.ea.resid = (uint16_t*)fz->x;
   }
   if (fast) {
     // router + shared gate/up; routed gate/up (one token: routing in its
@@ -684,6 +694,17 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
     HX_HIP(launch_down_dec(p.ea, s));
     if (T == 1) tm_ext_done(m, SLOT_DOWN);
     else tm_mark(m, SLOT_DOWN, 1, s);
+  } else if (few) {
+    if ((rc = run_routing(m, p, s))) return rc;
+    tm_ext(m, SLOT_GATE_UP, s);
+    HX_HIP(launch_gate_up_bf16(p.ea, s));
+    tm_ext_done(m, SLOT_GATE_UP);
+    tm_ext(m, SLOT_DOWN, s);
+    HX_HIP(launch_down_bf16(p.ea, s));
+    tm_ext_done(m, SLOT_DOWN);
+    tm_ext(m, SLOT_COMBINE, s);
+    HX_HIP(launch_combine_few(p.ea, s));
+    tm_ext_done(m, SLOT_COMBINE);
   } else if (decode) {
     // generic GEMVs; for GGUF weights every expert call (m = T <= 8) takes the
     // quantised arm: the tokens and then the rows of h as f32 d q of their Q8

@@ -52,6 +52,23 @@ HX_DEV void split3(float v, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   lo = __float_as_uint(r - __uint_as_float(ur & 0xffff0000u)) >> 16;
 }
 
+// the M tile of a workgroup. SM (up to HX_DECODE_MAX_T tokens): slot `tile` of the
+// decode plan, at most 8 rows; else the dispatch list's tile
+template <bool SM>
+HX_DEV bool bf_tile(const ExpertArgs& a, int tile, int& e, int& p0, int& rows) {
+  if constexpr (SM) {   // the record read together with the slot count
+    const int4 rec = *(const int4*)(a.plan + 4 + 4 * min(tile, a.max_slots - 1));
+    const int n = a.plan[0];
+    e = rec.x;
+    p0 = rec.y;
+    rows = rec.z;
+    return tile < n;
+  } else {
+    int mc;
+    return get_tile<HX_TILES_ALL>(a, tile, e, p0, rows, mc);
+  }
+}
+
 // the three planes of h: two in hbuf's bytes, one in hbf, rows of hstride
 HX_DEV uint16_t* h_plane(const ExpertArgs& a, int p) {
   return p < 2 ? (uint16_t*)a.hbuf + (int64_t)p * (a.F + a.T) * a.hstride : a.hbf;
@@ -65,7 +82,7 @@ HX_DEV uint16_t* h_plane(const ExpertArgs& a, int p) {
 constexpr int BG_K = 128, BG_LD = BG_K + 8;
 constexpr int BG_OP = 68;   // pitch of the f32 tile of h (aliases the rows)
 
-template <int MT>
+template <int MT, int LR>   // LR: rows an LDS buffer holds
 HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const uint8_t* G, const uint8_t* U, int rows, int p0,
                             int n0, bool sh) {
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, l16 = lane & 15, kq = lane >> 4;
@@ -96,7 +113,7 @@ HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const uint8_t* G,
   };
   auto store_a = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < MT; i++) *(u32x4_t*)(As + (buf * PM + r0 + 16 * i) * BG_LD + 8 * seg) = ar[i];
+    for (int i = 0; i < MT; i++) *(u32x4_t*)(As + (buf * LR + r0 + 16 * i) * BG_LD + 8 * seg) = ar[i];
   };
   f32x4_t acc[2][MT];
 #pragma unroll
@@ -121,7 +138,7 @@ HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const uint8_t* G,
     for (int s = 0; s < 4; s++) {
 #pragma unroll
       for (int i = 0; i < MT; i++) {
-        const bf16x8_t av = bfrag(As + (P * PM + 16 * i + l16) * BG_LD + 32 * s + 8 * kq);
+        const bf16x8_t av = bfrag(As + (P * LR + 16 * i + l16) * BG_LD + 32 * s + 8 * kq);
 #pragma unroll
         for (int m = 0; m < 2; m++) acc[m][i] = mfma_bf16(av, bfrag(b[P][m][s]), acc[m][i]);
       }
@@ -163,21 +180,27 @@ HX_DEV void bf_gate_up_main(const ExpertArgs& a, uint16_t* As, const uint8_t* G,
 }
 
 // grid (I / 64, tiles rounded up to 8), mapped by xcd_tile
-__global__ __launch_bounds__(256, 3) void k_gate_up_bf16(ExpertArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[2 * PM * BG_LD];
-  static_assert(sizeof(float) * PM * BG_OP <= sizeof(As), "the tile of h fits the rows' LDS");
-  int nt, tile, e, p0, rows, mc;
+template <bool SM>
+__global__ __launch_bounds__(256, SM ? 4 : 3) void k_gate_up_bf16(ExpertArgs a) {
+  constexpr int LR = SM ? 16 : PM;
+  __shared__ __attribute__((aligned(16))) uint16_t As[2 * LR * BG_LD];
+  static_assert(sizeof(float) * LR * BG_OP <= sizeof(As), "the tile of h fits the rows' LDS");
+  int nt, tile, e, p0, rows;
   xcd_tile(nt, tile);
-  if (!get_tile<HX_TILES_ALL>(a, tile, e, p0, rows, mc)) return;
+  if (!bf_tile<SM>(a, tile, e, p0, rows)) return;
   const bool sh = e == a.E;
   const uint8_t* G = sh ? a.sgate.base : a.gate.mat(e);
   const uint8_t* U = sh ? a.sup.base : a.up.mat(e);
   const int n0 = nt * 64;
-  switch ((rows + 15) >> 4) {   // uniform over the workgroup
-    case 1: bf_gate_up_main<1>(a, As, G, U, rows, p0, n0, sh); break;
-    case 2: bf_gate_up_main<2>(a, As, G, U, rows, p0, n0, sh); break;
-    case 3: bf_gate_up_main<3>(a, As, G, U, rows, p0, n0, sh); break;
-    default: bf_gate_up_main<4>(a, As, G, U, rows, p0, n0, sh); break;
+  if constexpr (SM) {
+    bf_gate_up_main<1, LR>(a, As, G, U, rows, p0, n0, sh);
+  } else {
+    switch ((rows + 15) >> 4) {   // uniform over the workgroup
+      case 1: bf_gate_up_main<1, LR>(a, As, G, U, rows, p0, n0, sh); break;
+      case 2: bf_gate_up_main<2, LR>(a, As, G, U, rows, p0, n0, sh); break;
+      case 3: bf_gate_up_main<3, LR>(a, As, G, U, rows, p0, n0, sh); break;
+      default: bf_gate_up_main<4, LR>(a, As, G, U, rows, p0, n0, sh); break;
+    }
   }
 }
 
@@ -187,15 +210,22 @@ __global__ __launch_bounds__(256, 3) void k_gate_up_bf16(ExpertArgs a) {
 // pieces of row r at slot piece ^ (r / 2 % 8) (rows are 128 bytes apart, so
 // without it every other row meets the same banks); the weights come 128 K at
 // a time. Rows are scaled by their routing weight by position and written as
-// bf16 to the per-assignment rows.
-constexpr int BD_K = 64, BD_PLANE = PM * BD_K, BD_STAGE = 3 * BD_PLANE;
-constexpr int BD_OP = 136;   // pitch of the bf16 output tile (aliases the rows)
+// bf16 to the per-assignment rows; SM (up to 8 tokens) as f32 ones, which
+// k_combine_few sums: the decode step's output is rounded once.
+constexpr int BD_K = 64;
+template <bool SM>
+struct Bd {
+  static constexpr int PLANE = (SM ? 32 : PM) * BD_K, STAGE = 3 * PLANE;
+};
+constexpr int BD_OP = 136;    // pitch of the bf16 output tile (aliases the rows)
+constexpr int BD_OPF = 132;   // of the f32 one
 
-template <int MT>
+template <int MT, bool SM>
 HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, float* rws, const uint8_t* W, int K, int rows, int p0, int n0,
                          float rw) {
   const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, l16 = lane & 15, kq = lane >> 4;
   constexpr int NA = (MT + 1) / 2;   // rounds of 32 rows
+  constexpr int BD_PLANE = Bd<SM>::PLANE, BD_STAGE = Bd<SM>::STAGE;
   const int nc = K / 128;            // even
   const uint8_t* bp = W + (int64_t)n0 * K * 2;
   const uint32_t bo = (uint32_t)((32 * wave + l16) * K + 8 * kq) * 2, bj = (uint32_t)(16 * K) * 2;
@@ -274,6 +304,19 @@ HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, float* rws, const ui
   step(nc - 1, ic<1>{}, ic<1>{}, ic<1>{});
   if (tid < PM) rws[tid] = rw;
   lds_barrier();
+  if constexpr (SM) {
+    float* of = (float*)As;
+    const f32x4_t w = *(const f32x4_t*)(rws + 4 * kq);
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) of[(4 * kq + q) * BD_OPF + 32 * wave + 16 * j + l16] = w[q] * acc[j][0][q];
+    lds_barrier();
+    const int m = tid >> 5, c4 = 4 * (tid & 31);   // rows 0 .. 7: a slot has no more
+    if (m < rows)
+      *(float4*)((float*)a.obuf + (int64_t)(p0 + m) * a.H + n0 + c4) = *(const float4*)(of + m * BD_OPF + c4);
+    return;
+  }
   uint16_t* ot = As;
 #pragma unroll
   for (int i = 0; i < MT; i++) {
@@ -293,24 +336,79 @@ HX_DEV void bf_down_main(const ExpertArgs& a, uint16_t* As, float* rws, const ui
 }
 
 // grid (H / 128, tiles rounded up to 8), mapped by xcd_tile
-__global__ __launch_bounds__(256, 3) void k_down_bf16(ExpertArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[2 * BD_STAGE];
+template <bool SM>
+__global__ __launch_bounds__(256, SM ? 4 : 3) void k_down_bf16(ExpertArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t As[2 * Bd<SM>::STAGE];
   __shared__ __attribute__((aligned(16))) float rws[PM];
-  static_assert(PM * BD_OP <= 2 * BD_STAGE, "the output tile fits the rows' LDS");
-  int nt, tile, e, p0, rows, mc;
+  static_assert(PM * BD_OP <= 2 * Bd<false>::STAGE && 16 * BD_OPF * 2 <= 2 * Bd<true>::STAGE,
+                "the output tile fits the rows' LDS");
+  int nt, tile, e, p0, rows;
   xcd_tile(nt, tile);
-  if (!get_tile<HX_TILES_ALL>(a, tile, e, p0, rows, mc)) return;
+  if (!bf_tile<SM>(a, tile, e, p0, rows)) return;
   const bool sh = e == a.E;
   const uint8_t* W = sh ? a.sdown.base : a.down.mat(e);
   const int K = sh ? a.Is : a.I, n0 = nt * 128;
   // a row's routing weight, used by the epilogue
   const float rw = threadIdx.x < PM ? a.wpos[p0 + min((int)threadIdx.x, rows - 1)] : 0.f;
-  switch ((rows + 15) >> 4) {   // uniform over the workgroup
-    case 1: bf_down_main<1>(a, As, rws, W, K, rows, p0, n0, rw); break;
-    case 2: bf_down_main<2>(a, As, rws, W, K, rows, p0, n0, rw); break;
-    case 3: bf_down_main<3>(a, As, rws, W, K, rows, p0, n0, rw); break;
-    default: bf_down_main<4>(a, As, rws, W, K, rows, p0, n0, rw); break;
+  if constexpr (SM) {
+    bf_down_main<1, SM>(a, As, rws, W, K, rows, p0, n0, rw);
+  } else {
+    switch ((rows + 15) >> 4) {   // uniform over the workgroup
+      case 1: bf_down_main<1, SM>(a, As, rws, W, K, rows, p0, n0, rw); break;
+      case 2: bf_down_main<2, SM>(a, As, rws, W, K, rows, p0, n0, rw); break;
+      case 3: bf_down_main<3, SM>(a, As, rws, W, K, rows, p0, n0, rw); break;
+      default: bf_down_main<4, SM>(a, As, rws, W, K, rows, p0, n0, rw); break;
+    }
   }
+}
+
+// ---------------------------------------------------------------- combine, up to 8 tokens
+// y[t] = the sum of token t's f32 rows in dispatch order (experts ascending, then
+// the shared expert), rounded once. Bound by latency: grid (T, H / 1024), four
+// outputs a thread, all its row loads together. RES as k_combine.
+template <bool RES>
+__global__ __launch_bounds__(256) void k_combine_few(ExpertArgs a) {
+  __shared__ int spos[HX_MAX_TOPK + 1];
+  const int t = blockIdx.x, k = a.k, tid = threadIdx.x;
+  if (tid < 64) {
+    const int p = tid < k ? a.inv[t * k + tid] : 0x7fffffff;
+    int rank = 0;
+    for (int j = 0; j < k; j++) rank += __builtin_amdgcn_readlane(p, j) < p;
+    if (tid < k) spos[rank] = p;
+    if (tid == 0) spos[k] = a.F + t;
+  }
+  const int n0 = (blockIdx.y * 256 + tid) * 4;
+  const bool in = n0 < a.H;
+  const int64_t o = (int64_t)t * a.H + (in ? n0 : 0);
+  uint2 rx = make_uint2(0u, 0u);
+  if (RES) rx = *(const uint2*)(a.resid + o);
+  __syncthreads();
+  if (!in) return;
+  const int nrows = k + (a.Is > 0 ? 1 : 0);
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  constexpr int B = 12;
+  for (int j0 = 0; j0 < nrows; j0 += B) {
+    float4 q[B];
+#pragma unroll
+    for (int j = 0; j < B; j++)   // past the last row: the last one again, not added
+      q[j] = *(const float4*)((const float*)a.obuf + (int64_t)spos[min(j0 + j, nrows - 1)] * a.H + n0);
+#pragma unroll
+    for (int j = 0; j < B; j++) {
+      const bool use = j0 + j < nrows;
+      acc[0] += use ? q[j].x : 0.f;
+      acc[1] += use ? q[j].y : 0.f;
+      acc[2] += use ? q[j].z : 0.f;
+      acc[3] += use ? q[j].w : 0.f;
+    }
+  }
+  uint32_t y[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    y[i] = f32_to_bf16(acc[i]);
+    const uint32_t w = i < 2 ? rx.x : rx.y;
+    if (RES) y[i] = f32_to_bf16(__uint_as_float(i & 1 ? w & 0xffff0000u : w << 16) + __uint_as_float(y[i] << 16));
+  }
+  *(uint2*)((RES ? a.resid : (uint16_t*)a.y) + o) = make_uint2(y[0] | (y[1] << 16), y[2] | (y[3] << 16));
 }
 
 // ---------------------------------------------------------------- launchers
@@ -318,18 +416,40 @@ __global__ __launch_bounds__(256, 3) void k_down_bf16(ExpertArgs a) {
 // column tiles divide; other widths take the GEMV kernels (from 9 tokens on the
 // MFMA kernels are the faster: 9 tokens 114 against 138 us, 301 tokens 365
 // against 1,856 us, 2048 tokens 777 against 12,660 us a forward of the 80B-A3B
-// layer)
+// layer; fewer tokens: few_bf16_ok)
 bool prefill_bf16_ok(const ExpertArgs& a) {
   return a.xbf && a.gate.fmt == HX_BF16 && a.down.fmt == HX_BF16 && a.H % 256 == 0 && a.I % 256 == 0 &&
          (a.Is == 0 || a.Is == a.I);
 }
 
+// A workgroup's K loop is a chain of round trips however few slots there are
+// (about 25 us over both launches), which the decode GEMVs' short workgroups do
+// not have: they stay the faster below five tokens or 30 assignments. Forward,
+// GEMV against this: 80B-A3B layer 3 tokens 69.8 / 58.4 us but 2 47.1 / 47.0, 4
+// 84.0 / 80.2, 5 101.8 / 90.2, 8 146.3 / 125.6; 128 experts of 256, hidden 2048,
+// top-8: 4 44.2 / 45.7, 5 52.4 / 49.2, 8 67.0 / 56.3; 128 of 768, top-6: 3
+// 51.9 / 58.3, 5 77.6 / 65.8, 8 105.0 / 74.0; 64 of 256, hidden 1024, top-4: 5
+// (20 assignments) 25.6 / 28.3, 6 28.7 / 29.8, 8 33.6 / 31.4.
+bool few_bf16_ok(const ExpertArgs& a) {
+  return a.T >= 5 && a.T <= HX_DECODE_MAX_T && a.T * a.k >= 30 && prefill_bf16_ok(a);
+}
+
 hipError_t launch_gate_up_bf16(const ExpertArgs& a, hipStream_t s) {
-  hx_launch(k_gate_up_bf16, dim3(a.I / 64, (a.max_tiles + 7) / 8 * 8), dim3(256), 0, s, a);
+  if (a.T <= HX_DECODE_MAX_T)
+    hx_launch(k_gate_up_bf16<true>, dim3(a.I / 64, (a.max_slots + 7) / 8 * 8), dim3(256), 0, s, a);
+  else hx_launch(k_gate_up_bf16<false>, dim3(a.I / 64, (a.max_tiles + 7) / 8 * 8), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 hipError_t launch_down_bf16(const ExpertArgs& a, hipStream_t s) {
-  hx_launch(k_down_bf16, dim3(a.H / 128, (a.max_tiles + 7) / 8 * 8), dim3(256), 0, s, a);
+  if (a.T <= HX_DECODE_MAX_T)
+    hx_launch(k_down_bf16<true>, dim3(a.H / 128, (a.max_slots + 7) / 8 * 8), dim3(256), 0, s, a);
+  else hx_launch(k_down_bf16<false>, dim3(a.H / 128, (a.max_tiles + 7) / 8 * 8), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+hipError_t launch_combine_few(const ExpertArgs& a, hipStream_t s) {
+  const dim3 g((unsigned)a.T, (unsigned)((a.H + 1023) / 1024));
+  if (a.resid) hx_launch(k_combine_few<true>, g, dim3(256), 0, s, a);
+  else hx_launch(k_combine_few<false>, g, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

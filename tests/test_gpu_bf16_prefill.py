@@ -11,7 +11,7 @@ of their magnitudes is below 4 max|y| over these inputs, so 5 * 2^-9 < 1e-2
 import pytest
 
 from oracle import oracle as O
-from tests.test_gpu_branches import TOL_BF16, Blk
+from tests.test_gpu_branches import TOL_BF16, Blk, x_np
 
 pytestmark = pytest.mark.gpu
 
@@ -24,3 +24,26 @@ def test_bf16_prefill_tiles(H, E, k, I, shared, norm, T):
     from helexa_amd import synth
     b = Blk(H, E, k, I, shared, norm, synth.FMT_BF16, O.BF16, 500 + H + E)
     b.check(b.x(T, seed=T), TOL_BF16, tag=f"bf16 prefill H{H} I{I} T={T}")
+
+
+# five to eight tokens (a slot's rows in one half-filled tile, f32 rows, one
+# rounding) and four, which stay on the decode GEMVs: slots of up to eight rows,
+# groups of eight slots partly filled, more rows a token than the combine holds
+# at a time
+@pytest.mark.parametrize("H,E,k,I,shared,norm", [(256, 8, 6, 256, 256, True), (2048, 64, 8, 512, 512, True),
+                                                 (1536, 9, 6, 768, 0, True), (768, 16, 14, 1024, 1024, False)])
+@pytest.mark.parametrize("T", [4, 5, 7, 8])
+def test_bf16_few_tokens(H, E, k, I, shared, norm, T):
+    import torch
+    from helexa_amd import synth
+    b = Blk(H, E, k, I, shared, norm, synth.FMT_BF16, O.BF16, 700 + H + E)
+    x = b.x(T, seed=T)
+    b.check(x, TOL_BF16, tag=f"bf16 few H{H} I{I} T={T}")
+    assert b.block.workspace_size(T) <= b.block.workspace_size(T + 1)
+    # the residual in the combine, and by itself for a stream off 16 bytes
+    w = torch.linspace(-0.5, 0.5, H, device="cuda")
+    n = torch.from_numpy(O.rmsnorm(x_np(x), w.cpu().numpy(), 1e-6, O.BF16)).to(torch.bfloat16)
+    ref = x.float() + b.block.forward(n.cuda().view_as(x)).float()
+    off = torch.empty(T * H + 8, dtype=x.dtype, device="cuda")[1:1 + T * H].view(T, H).copy_(x)
+    assert torch.equal(b.block.decoder_mlp_(x.clone(), w, 1e-6), b.block.decoder_mlp_(off, w, 1e-6))
+    assert torch.equal(off, ref.bfloat16())
