@@ -27,10 +27,13 @@
 // an XCD's four shader engines.
 //
 // MFMA (v_mfma_f32_16x16x32_f16: lane l holds A[l%16][8(l/16)+i],
-// B[8(l/16)+i][l%16], D rows 4(l/16)+i of column l%16) sums over K in any
-// order as long as A and B agree: step s of a chunk takes for lane group kq =
-// l / 16 the 8 elements at Frag::pos(s, kq), which is where the lane's own 16
-// bytes of codes lie, instead of 32 s + 8 kq.
+// B[8(l/16)+i][l%16], D rows 4(l/16)+i of column l%16): step s of a chunk takes
+// elements 32 s .. + 31, as in hx_prefill.hip, so that the partial sums, and with
+// them every output bit, are those of the kernels that dequantise into LDS.
+// Summing in the order in which the lanes' 16 bytes lie, without the exchange of
+// FragQ8::order, moved one output in 250 of a 512-token call by one bf16 step, for
+// 0.4 to 0.7 % of the time (512 tokens 252.0 us, 253.8 with it; 2048 445.7, 447.4);
+// 8-byte loads in place of the exchange took 314 and 573 us.
 #include "hx_prefill_dev.h"
 #include "hx_quant.h"
 #include <type_traits>
@@ -62,8 +65,9 @@ HX_DEV int swz(int i) { return (i & ~3) | ((i & 1) << 1) | ((i >> 1) & 1); }
 
 // ---------------------------------------------------------------- Q8_0
 // planar rows: K int8 codes, then the scale plane [rows][K / 32] f16. A lane
-// holds two runs of 16 codes a chunk: run u is elements 64 u + 16 kq .. + 15,
-// inside block 2 u + kq / 2 of the chunk. The scales of the tile's 128 weight
+// loads two runs of 16 codes a chunk: run u is piece m of elements 64 u .. + 63,
+// m = kq with its two bits exchanged, so that lane groups 2 j and 2 j + 1 hold
+// what either needs of steps 2 u and 2 u + 1 (order). The scales of the tile's 128 weight
 // rows are copied into LDS first, whole rows at a time: read chunk by chunk, 8
 // bytes of each row, every load touched 16 cache lines that were gone before
 // the next chunk's (2048 tokens of the 80B-A3B layer: gate/up 284 us, 215 us
@@ -79,8 +83,7 @@ struct FragQ8 {
   HX_HD static int aux_row(int K) { return (K < WIN ? K : WIN) / 16 + AUX_PAD; }
   __amdgpu_buffer_rsrc_t q;   // the matrix from the tile's first row on
   uint32_t qo;                // this lane's row
-  uint32_t sc;                // byte in aux of this lane's row's scale of block kq / 2
-  HX_DEV static int pos(int s, int kq) { return 64 * (s >> 1) + 16 * kq + 8 * (s & 1); }
+  uint32_t sc;                // byte in aux of this lane's row's scales
   // a weight row's scales in the plane behind a matrix of R rows
   HX_DEV static const uint8_t* aux_src(const uint8_t* mat, int R, int K, int row) {
     return mat + (int64_t)R * K + (int64_t)row * (K / 16);
@@ -112,23 +115,33 @@ struct FragQ8 {
   // rows row0 .. of a matrix; this lane's is row0 + r, its scales row ar of aux
   HX_DEV void init(const uint8_t* mat, int K, int row0, int r, int kq, int ar) {
     q = rsrc(mat + (int64_t)row0 * K, (uint32_t)(128 * K));   // at most 128 rows of a tile
-    qo = (uint32_t)(r * K + 16 * kq);
-    sc = (uint32_t)(ar * aux_row(K) + 2 * (kq >> 1));
+    qo = (uint32_t)(r * K + 16 * ((kq >> 1) | ((kq & 1) << 1)));
+    sc = (uint32_t)(ar * aux_row(K));
   }
   HX_DEV void load(int kc, Raw& w) const {
     w.q[0] = buf16(q, qo, (uint32_t)(kc * PD_K));
     w.q[1] = buf16(q, qo + 64, (uint32_t)(kc * PD_K));
   }
+  // run u as loaded -> its codes + 128, words 0, 1: elements 64 u + 8 kq .. + 7 (step 2 u), words
+  // 2, 3: 64 u + 32 + 8 kq .. (step 2 u + 1). permlane16_swap exchanges lane
+  // groups 1 and 3 of its first operand with 0 and 2 of its second.
+  HX_DEV static u32x4_t order(const Raw& w, int u) {
+    const u32x4_t c = w.q[u] ^ 0x80808080u;
+    const auto a = __builtin_amdgcn_permlane16_swap(c.x, c.z, false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(c.y, c.w, false, false);
+    return u32x4_t{a[0], b[0], a[1], b[1]};
+  }
+  // the scales of chunk kc of the window, a half a step
+  HX_DEV u32x2_t scales(int kc, const uint8_t* aux) const { return *(const u32x2_t*)(aux + sc + 8 * kc); }
   // MFMA operand of step s: (1024 + 128 + code) as f16 by the 0x64 byte, minus
   // 1152 (exact), times the scale (one rounding)
-  // of chunk kc of the window
-  HX_DEV f16x8_t frag(const Raw& w, int kc, int s, const uint8_t* aux) const {
-    const _Float16 sv = *(const _Float16*)(aux + sc + 8 * kc + 4 * (s >> 1));
+  HX_DEV static f16x8_t frag(u32x4_t run, int s, u32x2_t scales) {
+    const _Float16 sv = h2(scales[s >> 1])[s & 1];
     const h2_t sc2 = {sv, sv}, off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
     uint32_t o[4];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const uint32_t u = w.q[s >> 1][2 * (s & 1) + j] ^ 0x80808080u;
+      const uint32_t u = run[2 * (s & 1) + j];
       o[2 * j] = u32((h2(__builtin_amdgcn_perm(u, 0x64646464u, 0x00060004u)) + off) * sc2);
       o[2 * j + 1] = u32((h2(__builtin_amdgcn_perm(u, 0x64646464u, 0x00070005u)) + off) * sc2);
     }
@@ -194,15 +207,23 @@ HX_DEV void pd_gemm(uint8_t* lds, const F (&w)[PD_NF], int K, const uint8_t* asr
         load_b(kc + 1, ic<1 - P>{});
       }
       __builtin_amdgcn_sched_barrier(0);
+      u32x2_t sv[NF];
+      u32x4_t run[NF];   // not back into b: its next loads would be waited for here
+#pragma unroll
+      for (int f = 0; f < NF; f++) sv[f] = w[f].scales(kc, aux);
 #pragma unroll
       for (int s = 0; s < 4; s++) {
         f16x8_t bf[NF];
+        if (s % 2 == 0) {
 #pragma unroll
-        for (int f = 0; f < NF; f++) bf[f] = w[f].frag(b[P][f], kc, s, aux);
+          for (int f = 0; f < NF; f++) run[f] = F::order(b[P][f], s / 2);
+        }
+#pragma unroll
+        for (int f = 0; f < NF; f++) bf[f] = F::frag(run[f], s, sv[f]);
 #pragma unroll
         for (int i = 0; i < MT; i++) {
           const f16x8_t a =
-              __builtin_bit_cast(f16x8_t, ld16(As + (P * 16 * MT + 16 * i + l16) * PD_LD + F::pos(s, kq)));
+              __builtin_bit_cast(f16x8_t, ld16(As + (P * 16 * MT + 16 * i + l16) * PD_LD + 32 * s + 8 * kq));
 #pragma unroll
           for (int f = 0; f < NF; f++) acc[f][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bf[f], acc[f][i], 0, 0, 0);
         }
