@@ -2,7 +2,7 @@
 scale a 256-element run is the same weight in Q8_0 and in Q6_K, so beyond 64 rows
 an expert call, where both formats take f16 activations, the two blocks run the
 same products: the Q8_0 kernels (weights into registers) have to sum and round
-them as the kernels that dequantise into LDS do.
+them as the kernels that dequantise into LDS do, f16 h included (rounded once).
 Widths of one chunk pair, of several, and with more columns than the scales held
 in LDS at a time (2048); 16-row sub-tiles in every number and a remainder."""
 import numpy as np
@@ -52,8 +52,7 @@ def test_q8_prefill_bits(H, I, shared):
         return hx.Qwen3_5MoeBlock.load(cfg, out, act_dtype=hx.BF16)
 
     lds = block(hx.Q6_K, hx.Q6_K)
-    # gate and up Q6_K: the down products alone
-    regs = [(f, block(*f)) for f in ((hx.Q6_K, hx.Q8_0),)]
+    regs = [(f, block(*f)) for f in ((hx.Q8_0, hx.Q6_K), (hx.Q6_K, hx.Q8_0), (hx.Q8_0, hx.Q8_0))]
     for T in (65, 80, 97, 128, 300):
         x = synth.make_x(cfg, T, T)
         ref = lds.forward(x)
