@@ -241,7 +241,7 @@ inline bool hq_in_gate_up(const ExpertArgs& a) { return a.gate.fmt == HX_Q8_0 &&
 bool prefill_bf16_ok(const ExpertArgs& a);   // bf16 activations, bf16 experts: MFMA grouped GEMMs
 // 5 .. HX_DECODE_MAX_T tokens, bf16 experts: the same GEMMs over the decode
 // plan's slots, f32 rows and a combine of their own
-bool few_bf16_ok(const ExpertArgs& a);
+bool few_bf16_ok(const ExpertArgs& a, int64_t T);
 hipError_t launch_combine_few(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_gate_up_bf16(const ExpertArgs& a, hipStream_t s);
 hipError_t launch_down_bf16(const ExpertArgs& a, hipStream_t s);

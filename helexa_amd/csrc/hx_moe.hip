@@ -113,6 +113,9 @@ struct hx_moe {
   void* router = nullptr;
   float* rnorm = nullptr;   // [E1] |router row| rounded up (bf16 router rows only)
   WMat gate, up, down, sgate, sup, sdown;
+  ExpertArgs shape;   // widths and formats only: what picks a call's kernels
+  // [T]: the most workspace a call of up to T tokens takes
+  size_t small_ws[HX_DECODE_MAX_T + 1] = {};
   void* own_ws = nullptr;
   size_t own_ws_bytes = 0;
   Timing tm;
@@ -146,8 +149,7 @@ static ExpertArgs shape_args(const hx_moe* m) {
   return a;
 }
 static bool generic_path(const hx_moe* m, int64_t T) {
-  const ExpertArgs a = shape_args(m);
-  return T <= HX_DECODE_MAX_T ? !decode_fast_ok(a) : !prefill_mfma_ok(a);
+  return T <= HX_DECODE_MAX_T ? !decode_fast_ok(m->shape) : !prefill_mfma_ok(m->shape);
 }
 
 static WsLayout ws_layout(const hx_moe* m, int64_t T) {
@@ -180,13 +182,10 @@ static WsLayout ws_layout(const hx_moe* m, int64_t T) {
   L.hbuf = take(sizeof(float) * (F + T) * L.hstride);
   L.hbf = take(sizeof(uint16_t) * (F + T) * L.hstride);
   const size_t act = m->cfg.act_dtype == HX_BF16 ? 2 : 4;
-  ExpertArgs sa = shape_args(m);
-  sa.T = (int)T;
-  sa.k = (int)k;
-  const bool few = few_bf16_ok(sa);
+  const bool few = few_bf16_ok(m->shape, T), generic = generic_path(m, T);
+  const bool records = decode && !generic;   // what only the GGUF decode kernels use
   L.obuf = few ? take(sizeof(float) * (F + T) * H) : decode ? 0 : take(act * (F + T) * H);
   L.xh = decode ? 0 : take(sizeof(uint16_t) * T * H);
-  const bool generic = generic_path(m, T);
   // the MFMA path's xq lives in the routed rows of the weighted-rows buffer,
   // behind the router's logit planes: it is read by the gate/up kernels only,
   // before the down kernels write those rows (the shared expert's rows, which
@@ -196,14 +195,23 @@ static WsLayout ws_layout(const hx_moe* m, int64_t T) {
     L.xq = at + need <= act * F * H ? L.obuf + at : take(need);
   }
   L.xq32 = generic && gguf_fmt(m->gate.fmt) ? take(sizeof(float) * T * H) : 0;
-  L.xcv = decode && !few ? take(sizeof(uint32_t) * (size_t)T * (H / 32) * HX_XCV_WORDS) : 0;
-  L.hrec = decode && !few ? take(sizeof(uint32_t) * (size_t)(F + T) * ((I > Is ? I : Is) / 32) * HX_XCV_WORDS) : 0;
+  L.xcv = records ? take(sizeof(uint32_t) * (size_t)T * (H / 32) * HX_XCV_WORDS) : 0;
+  L.hrec = records ? take(sizeof(uint32_t) * (size_t)(F + T) * ((I > Is ? I : Is) / 32) * HX_XCV_WORDS) : 0;
   L.xn = take(act * T * H);
   L.ym = take(act * T * H);
-  L.dpart = decode && !few ? take(sizeof(float) * (size_t)down_groups((int)F, (int)T) * T * H) : 0;
+  L.dpart = records ? take(sizeof(float) * (size_t)down_groups((int)F, (int)T) * T * H) : 0;
   L.wpos = decode ? 0 : take(sizeof(float) * (F + T));
   L.total = o;
   return L;
+}
+
+// what a buffer for calls of T tokens holds: never less than a call of fewer
+// takes, so that a buffer sized once serves every smaller batch. Past
+// HX_DECODE_MAX_T tokens the layout grows with T; up to there it changes with the
+// kernels (records on GGUF experts, f32 weighted rows on bf16 ones) and may need
+// more than the smallest prefill layouts.
+static size_t ws_need(const hx_moe* m, int64_t T, const WsLayout& L) {
+  return std::max(L.total, m->small_ws[T < HX_DECODE_MAX_T ? T : HX_DECODE_MAX_T]);
 }
 
 // ----------------------------------------------------------------------------
@@ -404,16 +412,16 @@ extern "C" int hx_moe_create(const hx_moe_config* cfg, const hx_moe_weights* w, 
     hx_moe_destroy(m);
     return rc;
   }
+  m->shape = shape_args(m);
+  for (int T = 0; T <= HX_DECODE_MAX_T; T++)
+    m->small_ws[T] = std::max(ws_layout(m, T).total, T ? m->small_ws[T - 1] : 0);
   *out = m;
   return HX_OK;
 }
 
 extern "C" int hx_moe_workspace_size(const hx_moe* m, int64_t n_tokens, size_t* bytes) {
   if (!m || !bytes || n_tokens < 0) return fail(HX_ERR_INVALID_ARGUMENT, "bad argument");
-  // never less than a call of fewer tokens takes: up to HX_DECODE_MAX_T tokens on
-  // bf16 experts hold their weighted rows in f32, larger calls in bf16
-  const int64_t few = n_tokens < HX_DECODE_MAX_T ? n_tokens : HX_DECODE_MAX_T;
-  *bytes = std::max(ws_layout(m, n_tokens).total, ws_layout(m, few).total);
+  *bytes = ws_need(m, n_tokens, ws_layout(m, n_tokens));
   return HX_OK;
 }
 
@@ -526,7 +534,7 @@ static void make_plan(hx_moe* m, const void* x, int64_t T, void* y, uint8_t* ws,
   a.plan = d.plan;
   a.dpart = L.dpart ? (float*)(ws + L.dpart) : nullptr;
   // the plan holds the routing weights by position too
-  a.wpos = few_bf16_ok(a) ? (const float*)(d.plan + 4 + 4 * L.max_slots + F + T) : d.wpos;
+  a.wpos = few_bf16_ok(a, a.T) ? (const float*)(d.plan + 4 + 4 * L.max_slots + F + T) : d.wpos;
 }
 
 namespace hx {
@@ -650,7 +658,7 @@ static int forward_impl(hx_moe* m, const void* x, int64_t T, void* y, void* ws, 
   const bool bf = m->cfg.act_dtype == HX_BF16;
   const int H = m->cfg.hidden_size;
   uint16_t* xn = (uint16_t*)((uint8_t*)ws + L.xn);
-  const bool few = decode && !fast && few_bf16_ok(p.ea);
+  const bool few = decode && !fast && few_bf16_ok(p.ea, T);
   if (fz && fast && gguf_fmt(m->gate.fmt) && H <= 8 * 256) {
     // RMSNorm inside the router kernel (the router waves and the token-record
     // waves normalise each token with the same arithmetic, so both see the

@@ -430,8 +430,8 @@ bool prefill_bf16_ok(const ExpertArgs& a) {
 // top-8: 4 44.2 / 45.7, 5 52.4 / 49.2, 8 67.0 / 56.3; 128 of 768, top-6: 3
 // 51.9 / 58.3, 5 77.6 / 65.8, 8 105.0 / 74.0; 64 of 256, hidden 1024, top-4: 5
 // (20 assignments) 25.6 / 28.3, 6 28.7 / 29.8, 8 33.6 / 31.4.
-bool few_bf16_ok(const ExpertArgs& a) {
-  return a.T >= 5 && a.T <= HX_DECODE_MAX_T && a.T * a.k >= 30 && prefill_bf16_ok(a);
+bool few_bf16_ok(const ExpertArgs& a, int64_t T) {
+  return T >= 5 && T <= HX_DECODE_MAX_T && T * a.k >= 30 && prefill_bf16_ok(a);
 }
 
 hipError_t launch_gate_up_bf16(const ExpertArgs& a, hipStream_t s) {
