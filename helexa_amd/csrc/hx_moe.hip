@@ -437,15 +437,16 @@ static int get_ws(hx_moe* m, int64_t T, void*& ws, size_t& ws_bytes, WsLayout& L
     return HX_OK;
   }
   if (m->own_ws_bytes < L.total) {
+    const size_t need = ws_need(m, T, L);
     if (m->own_ws) {
       HX_HIP(hipDeviceSynchronize());
       (void)hipFree(m->own_ws);
       m->own_ws = nullptr;
       m->own_ws_bytes = 0;
     }
-    if (hipMalloc(&m->own_ws, L.total) != hipSuccess)
-      return fail(HX_ERR_OUT_OF_MEMORY, "workspace allocation of %zu bytes", L.total);
-    m->own_ws_bytes = L.total;
+    if (hipMalloc(&m->own_ws, need) != hipSuccess)
+      return fail(HX_ERR_OUT_OF_MEMORY, "workspace allocation of %zu bytes", need);
+    m->own_ws_bytes = need;
   }
   ws = m->own_ws;
   ws_bytes = m->own_ws_bytes;

@@ -32,3 +32,31 @@ def test_a_buffer_serves_smaller_calls(H, E, k, I, fmt):
         x = synth.make_x(b.cfg, T, T)
         ws = torch.empty(b.workspace_size(T + 1), dtype=torch.uint8, device="cuda")
         assert torch.equal(b.forward(x, workspace=ws), b.forward(x))
+
+
+@pytest.mark.parametrize("H,E,k,I,fmt", SHAPES)
+def test_own_workspace_serves_smaller_calls(H, E, k, I, fmt):
+    """the handle's own workspace, grown by a call of 9 tokens, holds every smaller
+    one: they can be captured (growing it is not possible there), and the replays
+    equal the eager results"""
+    from helexa_amd import synth
+    b = make(H, E, k, I, fmt)
+    xs = [synth.make_x(b.cfg, T, T) for T in (8, 7, 5)]
+    big = synth.make_x(b.cfg, 9, 9)
+    b.forward(big)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    outs, g = [torch.zeros_like(x) for x in xs], torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(g, stream=s):
+            for x, o in zip(xs, outs):
+                b.forward(x, stream=s, out=o)
+    torch.cuda.current_stream().wait_stream(s)
+    refs = [b.forward(x) for x in xs]
+    for _ in range(3):
+        for o in outs:
+            o.fill_(float("nan"))
+        b.forward(big)
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, r) for o, r in zip(outs, refs))
