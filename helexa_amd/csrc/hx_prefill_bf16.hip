@@ -41,15 +41,20 @@ template <int V>
 using ic = std::integral_constant<int, V>;
 
 // f32 -> bf16 parts hi, mid, lo with hi + mid + lo == v (each step truncates, so
-// the remainder is exact); inf and NaN go whole into hi
+// the remainder is exact); inf and NaN go whole into hi. A part that comes out
+// zero where v is not is the smallest bf16 of v's sign, 2^-133, instead: times an
+// infinite weight each part then gives the infinity that v gives, where a zero
+// gives NaN. What it adds to v is below half an f32 step from |v| = 2^-108 on.
 HX_DEV void split3(float v, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   const uint32_t u = __float_as_uint(v);
   const bool fin = (u & 0x7f800000u) != 0x7f800000u;
-  hi = v == v ? u >> 16 : 0x7fc0u;
   const float r = fin ? v - __uint_as_float(u & 0xffff0000u) : 0.f;
-  const uint32_t ur = __float_as_uint(r);
-  mid = ur >> 16;
-  lo = __float_as_uint(r - __uint_as_float(ur & 0xffff0000u)) >> 16;
+  const uint32_t ur = __float_as_uint(r), ul = __float_as_uint(r - __uint_as_float(ur & 0xffff0000u));
+  const uint32_t least = v == 0.f ? u >> 16 : ((u >> 16) & 0x8000u) | 1u;
+  auto part = [&](uint32_t w) { return w & 0x7fff0000u ? w >> 16 : least; };
+  hi = v == v ? part(u) : 0x7fc0u;
+  mid = part(ur);
+  lo = part(ul);
 }
 
 // the M tile of a workgroup. SM (up to HX_DECODE_MAX_T tokens): slot `tile` of the

@@ -47,3 +47,29 @@ def test_bf16_few_tokens(H, E, k, I, shared, norm, T):
     off = torch.empty(T * H + 8, dtype=x.dtype, device="cuda")[1:1 + T * H].view(T, H).copy_(x)
     assert torch.equal(b.block.decoder_mlp_(x.clone(), w, 1e-6), b.block.decoder_mlp_(off, w, 1e-6))
     assert torch.equal(off, ref.bfloat16())
+
+
+# h goes into the down products as three bf16 parts, of which some are exactly
+# zero: an infinite weight must still give the infinity that h itself gives.
+# Every output column of expert 0 meets one infinity, at another row of h
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("T", [7, 9, 130])
+def test_bf16_infinite_down_weights(T, sign):
+    import numpy as np
+    import torch
+    import helexa_amd as hx
+    from helexa_amd import synth
+    H, E, k, I = 1024, 8, 6, 256
+    cfg = hx.TextConfig(hidden_size=H, num_experts=E, num_experts_per_tok=k, moe_intermediate_size=I,
+                        shared_expert_intermediate_size=0, norm_topk_prob=True)
+    w = synth.make_weights(cfg, synth.FMT_BF16, 21)
+    n = torch.arange(H, device="cuda")
+    w["down"][1][0, n, n % I] = sign * float("inf")
+    b = hx.Qwen3_5MoeBlock.load(cfg, w, act_dtype=hx.BF16)
+    x = synth.make_x(cfg, T, 4)
+    got = b.forward(x).float().cpu().numpy()
+    ref = O.OracleMoe(H, E, k, I, 0, True, O.BF16, synth.to_numpy(w)).forward(x_np(x))
+    assert np.isinf(ref).any() and not np.isnan(ref).any()
+    fin = np.isfinite(ref)
+    assert np.array_equal(got[~fin], ref[~fin])
+    assert fin.any() and np.abs(got[fin] - ref[fin]).max() <= TOL_BF16 * np.abs(ref[fin]).max()
