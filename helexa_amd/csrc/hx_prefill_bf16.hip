@@ -413,7 +413,13 @@ __global__ __launch_bounds__(256) void k_combine_few(ExpertArgs a) {
     const uint32_t w = i < 2 ? rx.x : rx.y;
     if (RES) y[i] = f32_to_bf16(__uint_as_float(i & 1 ? w & 0xffff0000u : w << 16) + __uint_as_float(y[i] << 16));
   }
-  *(uint2*)((RES ? a.resid : (uint16_t*)a.y) + o) = make_uint2(y[0] | (y[1] << 16), y[2] | (y[3] << 16));
+  uint16_t* out = (RES ? a.resid : (uint16_t*)a.y) + o;
+  if (((uintptr_t)out & 7) == 0) {
+    *(uint2*)out = make_uint2(y[0] | (y[1] << 16), y[2] | (y[3] << 16));
+  } else {   // an output at any element, as the vector kernels take it
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[i] = (uint16_t)y[i];
+  }
 }
 
 // ---------------------------------------------------------------- launchers

@@ -73,3 +73,18 @@ def test_bf16_infinite_down_weights(T, sign):
     fin = np.isfinite(ref)
     assert np.array_equal(got[~fin], ref[~fin])
     assert fin.any() and np.abs(got[fin] - ref[fin]).max() <= TOL_BF16 * np.abs(ref[fin]).max()
+
+
+@pytest.mark.parametrize("offset", [1, 2, 4])
+def test_bf16_few_tokens_output_at_any_element(offset):
+    """an output that does not start on 8 bytes: same bits as one that does, and
+    nothing beside it written"""
+    import torch
+    from helexa_amd import synth
+    H, T = 768, 7
+    b = Blk(H, 16, 6, 256, 256, True, synth.FMT_BF16, O.BF16, 22)
+    x = b.x(T, seed=5)
+    buf = torch.full((T * H + 16,), 7.0, dtype=x.dtype, device="cuda")
+    out = buf[8 + offset:8 + offset + T * H].view(T, H)
+    assert torch.equal(b.block.forward(x, out=out), b.block.forward(x))
+    assert (buf[:8 + offset] == 7).all() and (buf[8 + offset + T * H:] == 7).all()
