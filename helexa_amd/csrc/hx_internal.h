@@ -19,6 +19,8 @@
 #define HX_DECODE_MAX_T 8
 // Rows of a grouped-GEMM M tile.
 #define HX_TILE_M 64
+// Workgroups along the second dimension of a grid (the device's limit).
+#define HX_MAX_GRID_Y 65536
 // Largest row count of an expert call that takes the reference's quantised
 // arm (activations quantised to the vec_dot type, integer block products):
 // QUANT_PREFILL_M_THRESHOLD (crates/neuron/src/harness/tp/tp_linear.rs:96);

@@ -427,9 +427,11 @@ __global__ __launch_bounds__(256) void k_combine_few(ExpertArgs a) {
 // column tiles divide; other widths take the GEMV kernels (from 9 tokens on the
 // MFMA kernels are the faster: 9 tokens 114 against 138 us, 301 tokens 365
 // against 1,856 us, 2048 tokens 777 against 12,660 us a forward of the 80B-A3B
-// layer; fewer tokens: few_bf16_ok)
+// layer; fewer tokens: few_bf16_ok). So do calls of more M tiles than a launch's
+// grid takes (from about 378,000 tokens of that layer on): the GEMV kernels' grids
+// do not grow with the tokens.
 bool prefill_bf16_ok(const ExpertArgs& a) {
-  return a.xbf && a.gate.fmt == HX_BF16 && a.down.fmt == HX_BF16 && a.H % 256 == 0 && a.I % 256 == 0 &&
+  return a.max_tiles <= HX_MAX_GRID_Y && a.xbf && a.gate.fmt == HX_BF16 && a.down.fmt == HX_BF16 && a.H % 256 == 0 && a.I % 256 == 0 &&
          (a.Is == 0 || a.Is == a.I);
 }
 
