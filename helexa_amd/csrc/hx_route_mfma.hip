@@ -539,7 +539,7 @@ __global__ __launch_bounds__(256) void k_route_mfma(RouterArgs a) {
       }
     }
     const float mx = route_logits_max<EPL>(v);
-    route_token_regs<EPL>(v, mx, k, a.norm, out_e, out_w);
+    route_token_regs<EPL>(v, mx, E, k, a.norm, out_e, out_w);
   }
   if (lane < k) {
     const int64_t f = (int64_t)t * k + lane;

@@ -107,9 +107,12 @@ HX_DEV int route_argmax(const float* v, float mx, int E) {
   return (int)~wave_max_u32(cand);
 }
 
-// softmax over the E logits of a token and this lane's keys, sorted
+// softmax over the E logits of a token and this lane's keys, sorted. Padding has
+// the key (0, ~e), which every expert's key is above, whatever its bits: a token
+// of NaN makes every quotient a NaN, of either sign (0 / NaN in the padding too),
+// and the ids of padding must not be selected for it.
 template <int EPL>
-HX_DEV void route_keys_from(float* v, float mx, uint32_t* h, uint32_t* l) {
+HX_DEV void route_keys_from(float* v, float mx, int E, uint32_t* h, uint32_t* l) {
   const int lane = lane_id();
 #pragma unroll
   for (int j = 0; j < EPL; j++) v[j] = v[j] - mx;
@@ -120,7 +123,7 @@ HX_DEV void route_keys_from(float* v, float mx, uint32_t* h, uint32_t* l) {
   s = wave_sum<64>(s);
 #pragma unroll
   for (int j = 0; j < EPL; j++) {
-    h[j] = __float_as_uint(v[j] / s);   // padding: 0 / s = +0
+    h[j] = lane + 64 * j < E ? __float_as_uint(v[j] / s) : 0u;
     l[j] = ~(uint32_t)(lane + 64 * j);
   }
   sort_keys_desc<EPL>(h, l);
@@ -129,7 +132,7 @@ template <int EPL>
 HX_DEV void route_keys(const float* lg, int E, uint32_t* h, uint32_t* l) {
   float v[EPL];
   const float mx = route_logits<EPL>(lg, E, v);
-  route_keys_from<EPL>(v, mx, h, l);
+  route_keys_from<EPL>(v, mx, E, h, l);
 }
 
 // One selection round: the wave-wide largest head probability m; when several
@@ -186,10 +189,10 @@ HX_DEV int route_round(uint32_t* h, uint32_t* l, uint32_t& pend, uint32_t& m) {
 // v: this lane's logits (expert lane + 64 j in v[j], padding -inf); mx: their
 // wave-wide maximum.
 template <int EPL>
-HX_DEV void route_token_regs(float* v, float mx, int k, bool norm, int& out_e, float& out_w) {
+HX_DEV void route_token_regs(float* v, float mx, int E, int k, bool norm, int& out_e, float& out_w) {
   const int lane = lane_id();
   uint32_t h[EPL], l[EPL];
-  route_keys_from<EPL>(v, mx, h, l);
+  route_keys_from<EPL>(v, mx, E, h, l);
   float my_p = 0.0f, tot = 0.0f;
   int my_e = 0;
   uint32_t pend = 0u;   // all-ones in the lane popped by the previous round
@@ -210,7 +213,7 @@ template <int EPL>
 HX_DEV void route_token_core(const float* lg, int E, int k, bool norm, int& out_e, float& out_w) {
   float v[EPL];
   const float mx = route_logits<EPL>(lg, E, v);
-  route_token_regs<EPL>(v, mx, k, norm, out_e, out_w);
+  route_token_regs<EPL>(v, mx, E, k, norm, out_e, out_w);
 }
 
 // route_token_core with K rounds unrolled and hook(r, e) called right after
@@ -241,7 +244,7 @@ HX_DEV void route_token_core_hook(float* v, int E, bool norm, int& out_e, float&
         hook(-1 - sp, e);
       }
     }
-    route_keys_from<EPL>(v, mx, h, l);
+    route_keys_from<EPL>(v, mx, E, h, l);
   }
   float my_p = 0.0f, tot = 0.0f;
   int my_e = 0;
