@@ -37,3 +37,28 @@ def test_quantiser_edges(dt, per_wg, blocks):
     got = out.cpu().numpy()
     assert np.array_equal(got[2:2 + ref.size], ref)
     assert not got[2 + ref.size:].any()
+
+
+@pytest.mark.parametrize("dt", [O.Q8_0, O.Q4_K, O.Q6_K, O.BF16, O.F16])
+def test_quantiser_special_values(dt):
+    """blocks with infinities, NaN, -0, denormals, values whose squares and sums
+    overflow or underflow, and blocks of nothing else"""
+    import torch
+    from helexa_amd import moe as hx
+    inf, nan = np.float32("inf"), np.float32("nan")
+    rng = np.random.default_rng(77)
+    special = [inf, -inf, nan, -0.0, 1e-45, -1e-40, 3e38, -3e38, 1e20, 1e-20, 2.0 ** -126, 65504.0, 70000.0]
+    x = rng.standard_normal((6 * len(special) + 4, 512)).astype(np.float32) * np.float32(0.02)
+    for i, v in enumerate(special):
+        x[6 * i, 5] = v                      # one in a block
+        x[6 * i + 1, 16:48] = v              # a run over sub-blocks
+        x[6 * i + 2, 256:] = v               # whole blocks
+        x[6 * i + 3, ::7] = v
+        x[6 * i + 4] *= v                    # a row scaled by it
+        x[6 * i + 5] = np.where(rng.random(512) < 0.5, v, -np.float32(v))
+    x[-4], x[-3], x[-2], x[-1] = 0.0, -0.0, nan, inf
+    x[-1, ::2] = -inf
+    ref = O.quantize(dt, x)
+    got = hx.quantize(dt, torch.from_numpy(x).cuda()).cpu().numpy()
+    bad = np.unique(np.nonzero(got.reshape(ref.shape) != ref)[0])
+    assert bad.size == 0, bad
