@@ -56,9 +56,8 @@ template <int FMT, int LPR, int CPL, int NTOK, int NRG>
 __global__ __launch_bounds__(256) void k_gate_up(ExpertArgs a) {
   using CK = Chunk<FMT>;
   constexpr int CH = CK::CH, RG = 64 / LPR, NS = CK::NSUM > 0 ? CK::NSUM : 1;
-  // the slot's record read together with the slot count (u < max_slots, so the
-  // record exists), and its first tokens' entries together with the weights:
-  // one round trip less each
+  // the slot's first tokens' entries are read together with the weights: one round
+  // trip less
   const int u = blockIdx.y;
   const int e = a.slots[3 * u], start = a.slots[3 * u + 1], count = a.slots[3 * u + 2];
   if (u >= a.counts[0]) return;

@@ -61,7 +61,7 @@ HX_DEV void split3(float v, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
 // decode plan, at most 8 rows; else the dispatch list's tile
 template <bool SM>
 HX_DEV bool bf_tile(const ExpertArgs& a, int tile, int& e, int& p0, int& rows) {
-  if constexpr (SM) {   // the record read together with the slot count
+  if constexpr (SM) {
     const int4 rec = *(const int4*)(a.plan + 4 + 4 * min(tile, a.max_slots - 1));
     const int n = a.plan[0];
     e = rec.x;
@@ -437,12 +437,13 @@ bool prefill_bf16_ok(const ExpertArgs& a) {
 
 // A workgroup's K loop is a chain of round trips however few slots there are
 // (about 25 us over both launches), which the decode GEMVs' short workgroups do
-// not have: they stay the faster below five tokens or 30 assignments. Forward,
-// GEMV against this: 80B-A3B layer 3 tokens 69.8 / 58.4 us but 2 47.1 / 47.0, 4
-// 84.0 / 80.2, 5 101.8 / 90.2, 8 146.3 / 125.6; 128 experts of 256, hidden 2048,
-// top-8: 4 44.2 / 45.7, 5 52.4 / 49.2, 8 67.0 / 56.3; 128 of 768, top-6: 3
+// not have. Forward, GEMV against this: 128 experts of 256, hidden 2048, top-8: 4
+// tokens 44.2 / 45.7 us, 5 52.4 / 49.2, 8 67.0 / 56.3; 128 of 768, top-6: 3
 // 51.9 / 58.3, 5 77.6 / 65.8, 8 105.0 / 74.0; 64 of 256, hidden 1024, top-4: 5
-// (20 assignments) 25.6 / 28.3, 6 28.7 / 29.8, 8 33.6 / 31.4.
+// (20 assignments) 25.6 / 28.3, 6 28.7 / 29.8, 8 33.6 / 31.4; 80B-A3B layer: 2
+// 47.1 / 47.0, 3 69.8 / 58.4, 4 84.0 / 80.2, 5 101.8 / 90.2, 8 146.3 / 125.6. The
+// line is where the smaller of these layers gain (five tokens, 30 assignments); the
+// widest would gain from 3 tokens on, which a rule on tokens alone gives up.
 bool few_bf16_ok(const ExpertArgs& a, int64_t T) {
   return T >= 5 && T <= HX_DECODE_MAX_T && T * a.k >= 30 && prefill_bf16_ok(a);
 }

@@ -31,9 +31,9 @@ HX_DEV bool get_tile(const ExpertArgs& a, int tile, int& e, int& p0, int& rows, 
     return true;
   }
   // the record's address needs no count (the grid is rounded up past the list's
-  // last record), so both can be read in one round trip; where the compiler
-  // moves the record behind the branch, tying the two together changed nothing
-  // (512 tokens Q4_K_M 210.8 / 210.7 us, 2048 Q8_0 434 / 433)
+  // last record). The compiler reads it behind the count's branch all the same;
+  // held together with the count it changed nothing (512 tokens Q4_K_M 210.8 /
+  // 210.7 us, 2048 Q8_0 434 / 433)
   const int4 rec = *(const int4*)(a.tiles + 4 * min(tile, a.max_tiles - 1));
   const int n = a.counts[1];
   m = rec.x;

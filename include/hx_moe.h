@@ -92,7 +92,8 @@ int hx_moe_create(const hx_moe_config* cfg, const hx_moe_weights* w, int device,
 /* Drop: frees the handle's device memory. NULL is accepted. */
 int hx_moe_destroy(hx_moe* m);
 
-/* Bytes of device workspace hx_moe_forward / hx_moe_route need for n_tokens. */
+/* Bytes of device workspace hx_moe_forward / hx_moe_route need for n_tokens or
+ * any fewer. */
 int hx_moe_workspace_size(const hx_moe* m, int64_t n_tokens, size_t* bytes);
 
 /* Module::forward (moe.rs:164-199 / tp_qwen3_5.rs:1240-1275), device resident:
